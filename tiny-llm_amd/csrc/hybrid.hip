@@ -17,6 +17,7 @@
 #include "common.h"
 #include "gemm8.h"
 #include "hybrid_kernels.h"
+#include "recur_chunk.h"
 #include "page_pool.h"
 
 #define HY_HIP(call)                                                                                   \
@@ -70,6 +71,7 @@ struct tl_hybrid {
     std::vector<float *> inv_freq;  // per mixer (2 layer + 0 / 1; those with rotary positions), device
     std::vector<float> rot_mult;    // per mixer: factor on cos and sin (rescaled frequencies)
     float *f32a = nullptr, *gates = nullptr, *idw = nullptr;  // [R, max_c] scratch (conv output, latent queries, channel decays); [R, H, 3]; [R]
+    float *chunk_ws = nullptr;                                 // chunked recurrences (recur_chunk.h): the largest layer's operands of every chunk of a step
     void *da = nullptr, *db = nullptr;                         // D-typed scratch rows: latents / low-rank inputs / attention read-out; plain queries
     hipStream_t stream = nullptr;
     bool owns_stream = false;
@@ -252,7 +254,42 @@ static int linear_t(const void *A, int lda, const void *W, float *out, int ldc, 
     return TL_OK;
 }
 
-static int launch_delta(const tl_hybrid *e, const tl_hybrid_layer &L, const MixState &run, const Meta &m, int n_seqs, const float *proj, int ldp) {
+// Recurrences of prompts in chunks of 64 tokens (recur_chunk.h): key widths with an instance of the kernels, on the float4 loads' alignment, from a chunk
+// length on that pays for two launches and a chunk's products (CHUNK_MIN, the longest sequence of the step; whole prompts of a 2048-wide Fonapel / Zefapel
+// list, token loop against chunks: 48 tokens 1,221 / 1,231 and 1,650 / 1,650 us, 128 tokens 1,098 / 1,071 and 1,483 / 1,448, 2,048 / 1,900 tokens
+// 2,988 / 2,195 and 3,149 / 2,616).  Key widths without an instance and decode steps stay with the token loop.
+constexpr int CHUNK_MIN = 48;
+static bool chunk_dims(const tl_hybrid_layer &L) { return (L.kind == TL_MIX_DELTA || L.kind == TL_MIX_LINREC) && (L.dim == 64 || L.dim == 128); }
+static int chunk_columns(const tl_hybrid_layer &L) { return (L.vdim + (L.kind == TL_MIX_LINREC && L.rec_kind == TL_REC_EXPGATE ? 1 : 0) + 15) / 16; }
+static size_t chunk_ws_floats(const tl_hybrid_layer &L, int rows, int slots) {
+    return chunk_dims(L) ? (size_t)(rows / CHUNK + slots + 1) * L.heads * ChunkLayout(L.dim, chunk_columns(L)).total : 0;
+}
+static bool chunk_takes(const tl_hybrid *e, const tl_hybrid_layer &L, const ChunkArgs &a, int max_len) {
+    return e->chunk_ws && max_len >= CHUNK_MIN && chunk_dims(L) && a.ld % 4 == 0 && a.q0 % 4 == 0 && a.k0 % 4 == 0 && (uintptr_t)a.src % 16 == 0;
+}
+static int launch_chunked(const tl_hybrid *e, const tl_hybrid_layer &L, ChunkArgs a, int kind, const Meta &m, int n_seqs, int max_len) {
+    a.ws = e->chunk_ws, a.obuf = e->obuf, a.seq_row0 = m.seq_row0, a.seq_slot = m.seq_slot, a.H = L.heads, a.vdim = L.vdim;
+    const dim3 prep(L.heads, n_seqs, (max_len + CHUNK - 1) / CHUNK), scan(L.heads, n_seqs, chunk_columns(L)), block(256);
+#define HY_CHUNK(KIND, DT)                                                              \
+    do {                                                                                \
+        hipLaunchKernelGGL((chunk_prep_kernel<KIND, DT>), prep, block, 0, e->stream, a); \
+        hipLaunchKernelGGL((chunk_scan_kernel<KIND, DT>), scan, block, 0, e->stream, a); \
+    } while (0)
+    if (L.dim == 128) {
+        if (kind == 0) HY_CHUNK(0, 8);
+        else if (kind == 1) HY_CHUNK(1, 8);
+        else HY_CHUNK(2, 8);
+    } else {
+        if (kind == 0) HY_CHUNK(0, 4);
+        else if (kind == 1) HY_CHUNK(1, 4);
+        else HY_CHUNK(2, 4);
+    }
+#undef HY_CHUNK
+    TL_CHECK_LAUNCH("hybrid chunked recurrence");
+    return TL_OK;
+}
+
+static int launch_delta(const tl_hybrid *e, const tl_hybrid_layer &L, const MixState &run, const Meta &m, int n_seqs, int max_len, const float *proj, int ldp) {
     // LPC lanes per state column with RPT key rows each: key_dim <= LPC * RPT.  The token loop is a dependency chain whose cost per wave hardly
     // depends on RPT, so the fewest lanes per column that still give every SIMD a wave: 64 while the step's columns are at most the SIMDs, then 32, then
     // a DPP row of 16 (also for narrow keys)
@@ -265,6 +302,10 @@ static int launch_delta(const tl_hybrid *e, const tl_hybrid_layer &L, const MixS
     dim3 grid(L.heads, n_seqs, (L.vdim + 256 / lpc - 1) / (256 / lpc)), block(256);
     const int C = conv_channels(L);
     const int a0 = 2 * L.kv_heads * L.dim + 2 * L.heads * L.vdim, b0 = a0 + L.heads;
+    ChunkArgs ca{};
+    ca.src = e->f32a, ca.ld = C, ca.q0 = 0, ca.k0 = L.kv_heads * L.dim, ca.v0 = 2 * L.kv_heads * L.dim, ca.group = L.heads / L.kv_heads;
+    ca.gate_src = proj, ca.ldg = ldp, ca.a0 = a0, ca.b0 = b0, ca.a_log = L.a_log_dev, ca.dt_bias = L.dt_bias_dev, ca.unit_eps = L.unit_eps, ca.state = run.state;
+    if (chunk_takes(e, L, ca, max_len)) return launch_chunked(e, L, ca, 0, m, n_seqs, max_len);
 #define HY_DELTA(RPT, LPC)                                                                                                                  \
     hipLaunchKernelGGL((delta_kernel<RPT, LPC>), grid, block, 0, e->stream, e->f32a, C, proj, ldp, a0, b0, L.a_log_dev, L.dt_bias_dev, \
                        L.unit_eps, m.seq_row0, m.seq_slot, run.state, e->obuf, L.heads, L.kv_heads, L.dim, L.vdim)
@@ -558,7 +599,7 @@ static int attention_talk(tl_hybrid *e, const tl_hybrid_layer &L, const void *kp
     return TL_OK;
 }
 
-static int launch_linrec(const tl_hybrid *e, const tl_hybrid_layer &L, const MixState &run, const Meta &m, int n_seqs, const float *proj, int ldp) {
+static int launch_linrec(const tl_hybrid *e, const tl_hybrid_layer &L, const MixState &run, const Meta &m, int n_seqs, int max_len, const float *proj, int ldp) {
     const bool chan = L.rec_kind == TL_REC_CHANNEL;
     const int ones = L.rec_kind == TL_REC_EXPGATE ? 1 : 0, VE = L.vdim + ones;
     // lanes per state column: a wave while the step's columns are few (decode), a DPP row of 16 otherwise (or for narrow keys)
@@ -575,6 +616,10 @@ static int launch_linrec(const tl_hybrid *e, const tl_hybrid_layer &L, const Mix
     const bool fixed = L.rec_kind == TL_REC_FIXED;
     const int silu = fixed && L.rec_silu ? (L.rot_dims > 0 ? 2 : 3) : 0;
     const float k_mul = fixed && L.rot_dims <= 0 && !L.rec_plain_k ? 1.f / sqrtf((float)L.dim) : 1.f;
+    ChunkArgs ca{};
+    ca.src = proj, ca.ld = ldp, ca.q0 = q0, ca.k0 = k0, ca.v0 = v0, ca.group = 1, ca.ones = ones, ca.state = run.state;
+    ca.gates = e->gates, ca.fixed = fixed ? L.decay_dev : nullptr, ca.silu = silu, ca.k_mul = k_mul, ca.decay = e->f32a;
+    if (chunk_takes(e, L, ca, max_len)) return launch_chunked(e, L, ca, chan ? 2 : 1, m, n_seqs, max_len);
 #define HY_LR(RPT, LPC, CHAN)                                                                                                                      \
     hipLaunchKernelGGL((linrec_kernel<RPT, LPC, CHAN>), grid, block, 0, e->stream, proj, ldp, q0, k0, v0, e->gates, e->f32a, m.seq_row0, m.seq_slot, \
                        run.state, e->obuf, L.heads, L.dim, L.vdim, ones, fixed ? L.decay_dev : (const float *)nullptr, silu, k_mul)
@@ -723,7 +768,7 @@ static int mixer_part_t(tl_hybrid *e, size_t ri, int part, float *proj, typename
                                    L.rec_plain_k ? 1.f : 1.f / sqrtf((float)L.dim), L.rec_silu, H, L.dim);
                 TL_CHECK_LAUNCH("hybrid constant decay prep");
             }
-            HY_TRY(launch_linrec(e, L, run, m, n_seqs, proj, ldp));
+            HY_TRY(launch_linrec(e, L, run, m, n_seqs, sh.max_len, proj, ldp));
             const int gate_kind = L.rec_sigmoid_gate ? 0 : 1;
             if (L.rec_joint_norm)
                 hipLaunchKernelGGL((linrec_out_joint_kernel<D>), dim3(rows), dim3(rows < 64 ? 1024 : 256), 0, st, e->obuf, L.out_norm_dev, c.norm_eps, proj + g0, ldp,
@@ -746,7 +791,7 @@ static int mixer_part_t(tl_hybrid *e, size_t ri, int part, float *proj, typename
                                m.seq_row0, m.seq_slot, run.conv_state, e->gates, H);
             TL_CHECK_LAUNCH("hybrid gate scan");
         }
-        HY_TRY(launch_linrec(e, L, run, m, n_seqs, proj, ldp));
+        HY_TRY(launch_linrec(e, L, run, m, n_seqs, sh.max_len, proj, ldp));
         hipLaunchKernelGGL((linrec_out_kernel<D>), dim3(rows, H), dim3(64), 0, st, e->obuf, L.vdim + (chan ? 0 : 1), chan ? 0 : 1, e->gates,
                            1.f / sqrtf((float)L.dim), L.out_norm_dev, chan ? 0 : L.vdim, c.norm_eps, proj + g0, ldp, chan ? 1 : 0, H, L.vdim, cat,
                            ldcat, out_scale);
@@ -763,7 +808,7 @@ static int mixer_part_t(tl_hybrid *e, size_t ri, int part, float *proj, typename
                            m.seq_row0, m.seq_slot, run.conv_state, n_seqs);
         TL_CHECK_LAUNCH("hybrid conv state");
     }
-    HY_TRY(launch_delta(e, L, run, m, n_seqs, proj, ldp));
+    HY_TRY(launch_delta(e, L, run, m, n_seqs, sh.max_len, proj, ldp));
     const float *gate = proj + (size_t)C;
     hipLaunchKernelGGL((delta_out_kernel<D>), dim3(rows, L.heads), dim3(64), 0, st, e->obuf, L.out_norm_dev, c.norm_eps, gate, ldp, L.heads,
                        L.vdim, cat, ldcat, out_scale);
@@ -1412,6 +1457,12 @@ extern "C" int tl_hybrid_create(const tl_hybrid_config *cfg, const tl_hybrid_lay
     HY_TRY(dev_alloc(p, &e->proj, (size_t)R * e->ld_proj));
     HY_TRY(dev_alloc(p, &e->qbuf, (size_t)R * std::max(1, max_q)));
     HY_TRY(dev_alloc(p, &e->f32a, (size_t)R * std::max(1, max_c)));
+    size_t chunk_floats = 0;
+    for (int i = 0; i < 2 * c.num_layers; ++i) {
+        const tl_hybrid_layer &L = i % 2 ? e->beside[i / 2] : e->layers[i / 2];
+        if (R >= CHUNK_MIN && L.kind >= 0) chunk_floats = std::max(chunk_floats, chunk_ws_floats(L, R, c.max_slots));
+    }
+    if (chunk_floats) HY_TRY(dev_alloc(p, &e->chunk_ws, chunk_floats));
     HY_TRY(dev_alloc(p, &e->gates, (size_t)R * max_gh * 3));
     HY_TRY(dev_alloc(p, &e->idw, (size_t)R));
     HY_TRY(dev_alloc(p, (char **)&e->da, (size_t)R * max_da * es));
