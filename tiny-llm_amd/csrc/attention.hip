@@ -7,6 +7,12 @@
 #include "common.h"
 #include "kv8.h"
 
+#define TL_TRY(expr)                  \
+    do {                              \
+        const int rc_ = (expr);       \
+        if (rc_ != TL_OK) return rc_; \
+    } while (0)
+
 namespace tl {
 
 constexpr float LOG2E = 1.44269504089f;
@@ -406,14 +412,24 @@ __device__ __forceinline__ void fa_sload_i32(const int32_t *ptr, int &dst) { asm
 __device__ __forceinline__ void fa_sload_wait(int &a) { asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(a)); }
 constexpr int FA_KS_ELEMS = FA_BK * 128, FA_VS_ELEMS = FA_BK * FA_VROW;
 constexpr size_t fa_pipe_lds_bytes() { return (size_t)2 * (FA_KS_ELEMS + FA_VS_ELEMS) * 2 + 2 * FA_BK * sizeof(int); }
-template <bool ONEPAGE, int QR = 1, bool KV8 = false, int NW = 4>
+// SEQS = PackedSeqs: several sequences of unequal length in one launch (grid z), q and out in row order [row][head][128] -- the order the projections around
+// it read and write.  A short prompt alone fills a fraction of the chip: six of 333 ... 84 tokens took 6 x 17 us a layer one after another (and 6 x 10 us for
+// their preparation and the heads' way back to rows), 34 us together.
+struct OneShape {};
+template <bool ONEPAGE, int QR = 1, bool KV8 = false, int NW = 4, typename SEQS = OneShape>
 __global__ __launch_bounds__(64 * NW, (QR == 1 && NW == 4) ? 2 : 1) void paged_fa_bf16_d128_kernel(
     const uint16_t *__restrict__ q, const void *__restrict__ key_pages_v, const void *__restrict__ value_pages_v,
     const int32_t *__restrict__ block_table, const int32_t *__restrict__ context_lens, uint16_t *__restrict__ out,
-    float *__restrict__ ws, int n_splits, int L, int page_size, int page_shift, int max_pages, int num_heads, int num_kv_heads,
-    float scale, int is_causal, int xcd_remap, const float *__restrict__ key_scales = nullptr,
-    const float *__restrict__ value_scales = nullptr) {
+    float *__restrict__ ws, int n_splits, int L_arg, int page_size, int page_shift, int max_pages, int num_heads, int num_kv_heads,
+    float scale, int is_causal, int xcd_remap, const float *__restrict__ key_scales, const float *__restrict__ value_scales, const SEQS seqs) {
     constexpr int D = 128;
+    constexpr bool PACKED = !std::is_same<SEQS, OneShape>::value;
+    int L = L_arg, b = blockIdx.z, row0 = 0, ctx;  // b: the sequence's row of the block table
+    if constexpr (PACKED) {
+        L = seqs.len[blockIdx.z], b = seqs.slot[blockIdx.z], row0 = seqs.row0[blockIdx.z], ctx = seqs.ctx[blockIdx.z];
+    } else {
+        ctx = context_lens[b];
+    }
     using KVE = typename std::conditional<KV8, uint8_t, uint16_t>::type;  // a page element
     using KVC = typename std::conditional<KV8, u32x2, u32x4>::type;        // a chunk of 8 of them
     const KVE *__restrict__ key_pages = reinterpret_cast<const KVE *>(key_pages_v);
@@ -447,7 +463,6 @@ __global__ __launch_bounds__(64 * NW, (QR == 1 && NW == 4) ? 2 : 1) void paged_f
         kvh = t / gx;
         bx = t - kvh * gx;
     }
-    const int b = blockIdx.z;
     const int rep = num_heads / num_kv_heads;
     const int QB = (L + 32 * QR - 1) / (32 * QR);  // query blocks of 32 QR rows: one per wave
     const int items = rep * QB;
@@ -455,13 +470,15 @@ __global__ __launch_bounds__(64 * NW, (QR == 1 && NW == 4) ? 2 : 1) void paged_f
     // range is cut into n_splits pieces, one workgroup each, merged by paged_merge_kernel (flash-decoding style)
     const int split = bx % n_splits;
     // causal chunks: the LAST query blocks see the most tokens -- they go first (launch order = dispatch order), the light ones fill the tail
-    const int item_block = is_causal ? ((int)gridDim.x / n_splits - 1 - bx / n_splits) : bx / n_splits;
+    const int item_blocks = PACKED ? (items + NW - 1) / NW : (int)gridDim.x / n_splits;
+    if (PACKED && bx / n_splits >= item_blocks) return;  // (the grid is as wide as the longest sequence needs)
+    const int item_block = is_causal ? (item_blocks - 1 - bx / n_splits) : bx / n_splits;
     const int item = item_block * NW + wave;
     const bool wave_live = item < items;
     const int hq = wave_live ? item % rep : 0;
     const int qb = wave_live ? item / rep : 0;
     const int n = b * num_heads + kvh * rep + hq;
-    const int ctx = context_lens[b];
+    auto row_of = [&](int t) { return PACKED ? (long)(row0 + t) * num_heads + kvh * rep + hq : (long)n * L + t; };  // row of q, out and the partials
     const float scale_log2 = scale * LOG2E;
     int qrow[QR];
     bool q_valid[QR];
@@ -476,7 +493,7 @@ __global__ __launch_bounds__(64 * NW, (QR == 1 && NW == 4) ? 2 : 1) void paged_f
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
             if (q_valid[rb]) {
-                qf[rb][s] = *reinterpret_cast<const u32x4 *>(q + ((long)n * L + qrow[rb]) * D + 16 * s + 8 * h);
+                qf[rb][s] = *reinterpret_cast<const u32x4 *>(q + row_of(qrow[rb]) * D + 16 * s + 8 * h);
             } else {
                 qf[rb][s] = u32x4{0u, 0u, 0u, 0u};
             }
@@ -833,7 +850,7 @@ __global__ __launch_bounds__(64 * NW, (QR == 1 && NW == 4) ? 2 : 1) void paged_f
         if (!q_valid[rb]) continue;
         if (n_splits > 1) {
             // un-normalised partial: D values, running max (log2 domain), running sum
-            float *w = ws + (((long)n * L + qrow[rb]) * n_splits + split) * (D + 2);
+            float *w = ws + (row_of(qrow[rb]) * n_splits + split) * (D + 2);
 #pragma unroll
             for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -846,7 +863,7 @@ __global__ __launch_bounds__(64 * NW, (QR == 1 && NW == 4) ? 2 : 1) void paged_f
             }
             continue;
         }
-        uint16_t *orow = out + ((long)n * L + qrow[rb]) * D;
+        uint16_t *orow = out + row_of(qrow[rb]) * D;
         const float inv = run_sum[rb] == 0.f ? 0.f : 1.0f / run_sum[rb];
 #pragma unroll
         for (int db = 0; db < 4; ++db) {
@@ -968,6 +985,45 @@ extern "C" size_t tl_paged_attention_workspace_bytes(int N, int L, int D, int pa
     return (size_t)N * L * splits * (D + 2) * sizeof(float);
 }
 
+struct FaLaunch {
+    const uint16_t *q;
+    const void *key_pages, *value_pages;
+    const float *key_scales, *value_scales;
+    const int32_t *block_table, *context_lens;
+    uint16_t *out;
+    float *ws;
+    int splits, L, page_size, page_shift, max_pages, num_heads, num_kv_heads;
+    float scale;
+    int is_causal;
+};
+template <bool ONEP, bool K8, int NW, typename SEQS>
+static int launch_fa_instance(const FaLaunch &f, dim3 grid, const SEQS &seqs, hipStream_t st) {
+    const auto kernel = paged_fa_bf16_d128_kernel<ONEP, 1, K8, NW, SEQS>;
+    const size_t lds = NW == 8 ? fa_pipe_lds_bytes() : 0;
+    if (NW == 8) {
+        static bool attr_set_dev[64] = {};  // per HIP device: a function attribute belongs to the device's code object
+        int dev = 0;
+        (void)hipGetDevice(&dev);
+        bool &attr_set = attr_set_dev[dev & 63];
+        if (!attr_set) {
+            if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+                return fail(TL_ERR_HIP, "paged_attention: cannot size the prefill kernel's LDS");
+            attr_set = true;
+        }
+    }
+    const int xcd_remap = 1;  // one KV head per XCD (+2 % at 8k prefill)
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, st, f.q, f.key_pages, f.value_pages, f.block_table, f.context_lens, f.out, f.ws, f.splits, f.L, f.page_size,
+                       f.page_shift, f.max_pages, f.num_heads, f.num_kv_heads, f.scale, f.is_causal, xcd_remap, f.key_scales, f.value_scales, seqs);
+    return TL_OK;
+}
+// w8: 8 waves sharing a double-buffered tile (pages of 64+ tokens); else 4, with the one-page form where a 64-token stage never straddles pages
+template <typename SEQS>
+static int launch_fa(const FaLaunch &f, dim3 grid, bool w8, bool kv8, const SEQS &seqs, hipStream_t st) {
+    if (w8) return kv8 ? launch_fa_instance<true, true, 8>(f, grid, seqs, st) : launch_fa_instance<true, false, 8>(f, grid, seqs, st);
+    if (f.page_shift >= 6) return kv8 ? launch_fa_instance<true, true, 4>(f, grid, seqs, st) : launch_fa_instance<true, false, 4>(f, grid, seqs, st);
+    return kv8 ? launch_fa_instance<false, true, 4>(f, grid, seqs, st) : launch_fa_instance<false, false, 4>(f, grid, seqs, st);
+}
+
 // key_scales != nullptr: FP8 pages (bf16 queries, head dimension 128)
 static int paged_attention_impl(const void *q, const void *key_pages, const void *value_pages, const float *key_scales,
                                 const float *value_scales, const int32_t *block_table, const int32_t *context_lens, void *out, int N,
@@ -1011,39 +1067,12 @@ static int paged_attention_impl(const void *q, const void *key_pages, const void
         const size_t fa_need = fa_splits > 1 ? (size_t)N * L * fa_splits * (D + 2) * sizeof(float) : 0;
         if (fa_need > 0 && (!workspace || workspace_bytes < fa_need)) fa_splits = 1;  // no workspace: one pass, still correct
         const dim3 grid(item_blocks * fa_splits, num_kv_heads, B);
-        const int fa_xcd_remap = 1;  // one KV head per XCD (round 3 A/B: +2 % at 8k prefill)
-#define FA_LAUNCH(ONEP, QRv, K8)                                                                                                \
-        hipLaunchKernelGGL((paged_fa_bf16_d128_kernel<ONEP, QRv, K8>), grid, dim3(256), 0, st, (const uint16_t *)q, key_pages,  \
-                           value_pages, block_table, context_lens, (uint16_t *)out, (float *)workspace, fa_splits, L, page_size, \
-                           page_shift, max_pages, num_heads, num_kv_heads, scale, is_causal, fa_xcd_remap, key_scales,            \
-                           value_scales)
-#define FA_LAUNCH8(K8)                                                                                                           \
-        do {                                                                                                                         \
-            static bool attr_set_dev[64] = {};  /* per HIP device: a function attribute belongs to the device's code object */      \
-            int dev_ = 0;                                                                                                            \
-            (void)hipGetDevice(&dev_);                                                                                               \
-            bool &attr_set = attr_set_dev[dev_ & 63];                                                                                \
-            if (!attr_set) {                                                                                                         \
-                if (hipFuncSetAttribute(reinterpret_cast<const void *>(&paged_fa_bf16_d128_kernel<true, 1, K8, 8>),                  \
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)fa_pipe_lds_bytes()) != hipSuccess)         \
-                    return fail(TL_ERR_HIP, "paged_attention: cannot size the prefill kernel's LDS");                               \
-                attr_set = true;                                                                                                     \
-            }                                                                                                                        \
-            hipLaunchKernelGGL((paged_fa_bf16_d128_kernel<true, 1, K8, 8>), grid, dim3(512), fa_pipe_lds_bytes(), st,                \
-                               (const uint16_t *)q, key_pages, value_pages, block_table, context_lens, (uint16_t *)out,             \
-                               (float *)workspace, fa_splits, L, page_size, page_shift, max_pages, num_heads, num_kv_heads, scale,   \
-                               is_causal, fa_xcd_remap, key_scales, value_scales);                                                   \
-        } while (0)
-        if (w8) {
-            if (kv8) FA_LAUNCH8(true);
-            else FA_LAUNCH8(false);
-        } else if (kv8) {
-            if (page_shift >= 6) FA_LAUNCH(true, 1, true);
-            else FA_LAUNCH(false, 1, true);
-        } else if (page_shift >= 6) FA_LAUNCH(true, 1, false);  // a 64-token stage never straddles pages
-        else FA_LAUNCH(false, 1, false);
-#undef FA_LAUNCH
-#undef FA_LAUNCH8
+        FaLaunch f{};
+        f.q = (const uint16_t *)q, f.key_pages = key_pages, f.value_pages = value_pages, f.key_scales = key_scales, f.value_scales = value_scales;
+        f.block_table = block_table, f.context_lens = context_lens, f.out = (uint16_t *)out, f.ws = (float *)workspace, f.splits = fa_splits, f.L = L;
+        f.page_size = page_size, f.page_shift = page_shift, f.max_pages = max_pages, f.num_heads = num_heads, f.num_kv_heads = num_kv_heads;
+        f.scale = scale, f.is_causal = is_causal;
+        TL_TRY(launch_fa(f, grid, w8, kv8, OneShape{}, st));
         TL_CHECK_LAUNCH("paged_attention(prefill)");
         if (fa_splits > 1) {
             hipLaunchKernelGGL((paged_merge_kernel<BF16>), dim3(N * L), dim3(128), 0, st, (const float *)workspace,
@@ -1104,6 +1133,40 @@ extern "C" int tl_paged_attention(const void *q, const void *key_pages, const vo
     return paged_attention_impl(q, key_pages, value_pages, nullptr, nullptr, block_table, context_lens, out, N, L, D, num_pages, page_size,
                                 max_pages, num_heads, num_kv_heads, scale, is_causal, max_context_hint, dtype, workspace, workspace_bytes,
                                 stream);
+}
+
+int tl::paged_attention_packed(const uint16_t *q, const void *key_pages, const void *value_pages, const float *key_scales, const float *value_scales,
+                               const int32_t *block_table, uint16_t *out, const PackedSeqs &seqs, int page_size, int max_pages, int num_heads, int num_kv_heads,
+                               float scale, float *workspace, size_t workspace_bytes, hipStream_t stream) {
+    TL_REQUIRE(seqs.n >= 1 && seqs.n <= PACK_MAX, "paged_attention_packed: between 1 and 16 sequences");
+    const int rep = num_heads / num_kv_heads;
+    FaLaunch f{};
+    f.page_shift = -1;
+    for (int sh = 0; sh < 30; ++sh)
+        if ((1 << sh) == page_size) f.page_shift = sh;
+    int longest = 0, rows = 0, max_ctx = 0;
+    for (int i = 0; i < seqs.n; ++i)
+        longest = std::max(longest, seqs.len[i]), rows = std::max(rows, seqs.row0[i] + seqs.len[i]), max_ctx = std::max(max_ctx, seqs.ctx[i]);
+    const bool w8 = g_fa_waves == 8 && f.page_shift >= 6 && longest >= 64;
+    const int nw = w8 ? 8 : 4;
+    int blocks = 0;  // of all sequences
+    for (int i = 0; i < seqs.n; ++i) blocks += (rep * ((seqs.len[i] + 31) / 32) + nw - 1) / nw;
+    const int widest = (rep * ((longest + 31) / 32) + nw - 1) / nw;
+    int splits = pick_fa_splits(1, num_kv_heads, blocks, max_ctx, w8 ? 256 : 512);
+    if (splits > 1 && (!workspace || workspace_bytes < (size_t)rows * num_heads * splits * (128 + 2) * sizeof(float))) splits = 1;
+    f.q = q, f.key_pages = key_pages, f.value_pages = value_pages, f.key_scales = key_scales, f.value_scales = value_scales, f.block_table = block_table;
+    f.out = out, f.ws = workspace, f.splits = splits, f.page_size = page_size, f.max_pages = max_pages, f.num_heads = num_heads, f.num_kv_heads = num_kv_heads;
+    f.scale = scale, f.is_causal = 1;
+    TL_TRY(launch_fa(f, dim3(widest * splits, num_kv_heads, seqs.n), w8, key_scales != nullptr, seqs, stream));
+    TL_CHECK_LAUNCH("paged_attention(packed prefill)");
+    if (splits > 1) {
+        for (int i = 0; i < seqs.n; ++i) {  // (rows of the pass that no sequence of the launch owns are not touched)
+            const size_t row = (size_t)seqs.row0[i] * num_heads;
+            hipLaunchKernelGGL((paged_merge_kernel<BF16>), dim3(seqs.len[i] * num_heads), dim3(128), 0, stream, workspace + row * splits * (128 + 2), out + row * 128, 128, splits);
+        }
+        TL_CHECK_LAUNCH("paged_attention(packed prefill merge)");
+    }
+    return TL_OK;
 }
 
 // ---- FP8 (E4M3) KV pages: the quantised twins of paged_cache_update / paged_attention (kv8.h, include/tinyllm_hip.h) ----------------

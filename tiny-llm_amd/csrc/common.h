@@ -203,6 +203,17 @@ __device__ __forceinline__ void prof_end(prof_t *buf, prof_t t0) {
     }
 }
 
+// Several sequences' rows side by side in one pass: sequence i holds rows row0[i] .. row0[i] + len[i] of the pass, is row slot[i] of the block table and is
+// ctx[i] tokens long behind the pass.
+constexpr int PACK_MAX = 16;
+struct PackedSeqs {
+    int n, row0[PACK_MAX], len[PACK_MAX], slot[PACK_MAX], ctx[PACK_MAX];
+};
+// attention.hip: causal FlashAttention of several sequences in one launch, q and out in row order [row][head][128]
+int paged_attention_packed(const uint16_t *q, const void *key_pages, const void *value_pages, const float *key_scales, const float *value_scales,
+                           const int32_t *block_table, uint16_t *out, const PackedSeqs &seqs, int page_size, int max_pages, int num_heads, int num_kv_heads,
+                           float scale, float *workspace, size_t workspace_bytes, hipStream_t stream);
+
 inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 
 }  // namespace tl

@@ -1871,12 +1871,59 @@ static void launch_qkv_post(tl_engine *e, int l, QkvPostArgs &q, int n) {
     q.value_scales = e->layer_vs(l);
     switch (e->cfg.head_dim) {
         case 128:
-            if (e->kv_format == TL_KV_FP8_E4M3) hipLaunchKernelGGL((qkv_post_kernel<8, true>), dim3(n), dim3(256), 0, e->stream, q);
-            else hipLaunchKernelGGL((qkv_post_kernel<8>), dim3(n), dim3(256), 0, e->stream, q);
+            if (e->kv_format == TL_KV_FP8_E4M3) hipLaunchKernelGGL((qkv_post_kernel<8, true>), dim3(n), dim3(256), 0, e->stream, q, OneSeq{});
+            else hipLaunchKernelGGL((qkv_post_kernel<8>), dim3(n), dim3(256), 0, e->stream, q, OneSeq{});
             break;
-        case 64: hipLaunchKernelGGL((qkv_post_kernel<4>), dim3(n), dim3(256), 0, e->stream, q); break;
-        default: hipLaunchKernelGGL((qkv_post_kernel<2>), dim3(n), dim3(256), 0, e->stream, q); break;
+        case 64: hipLaunchKernelGGL((qkv_post_kernel<4>), dim3(n), dim3(256), 0, e->stream, q, OneSeq{}); break;
+        default: hipLaunchKernelGGL((qkv_post_kernel<2>), dim3(n), dim3(256), 0, e->stream, q, OneSeq{}); break;
     }
+}
+
+// Head norms, RoPE and K/V append of every row of a pass, then its attention: attn [rows][Hq * 128].  Sequences of more than 8 tokens share one launch of the
+// FlashAttention kernel; shorter ones take the decode kernel (float32 weights), one after another.  head_dim 128.
+static int prefill_attention(tl_engine *e, int l, const PackedSeqs &seqs, int rows) {
+    const tl_engine_config &c = e->cfg;
+    const tl_layer_weights &w = e->layers[l];
+    const int D = c.head_dim, Hq = c.num_heads, Hkv = c.num_kv_heads;
+    const bool kv8 = e->kv_format == TL_KV_FP8_E4M3;
+    QkvPostArgs q{};
+    q.qkv = e->qkv;
+    q.q_norm_w = (const uint16_t *)w.q_norm_dev;
+    q.k_norm_w = (const uint16_t *)w.k_norm_dev;
+    q.q_t = e->q_t;
+    q.key_pages = e->layer_k(l);
+    q.value_pages = e->layer_v(l);
+    q.key_scales = e->layer_ks(l);
+    q.value_scales = e->layer_vs(l);
+    q.block_row = e->block_table;
+    q.page_size = c.page_size;
+    q.max_pages = c.max_pages_per_seq;
+    q.num_heads = Hq;
+    q.num_kv_heads = Hkv;
+    q.eps = c.rms_norm_eps;
+    q.rope_base = c.rope_theta;
+    if (kv8) hipLaunchKernelGGL((qkv_post_kernel<8, true, PackedSeqs>), dim3(rows), dim3(256), 0, e->stream, q, seqs);
+    else hipLaunchKernelGGL((qkv_post_kernel<8, false, PackedSeqs>), dim3(rows), dim3(256), 0, e->stream, q, seqs);
+    TL_CHECK_LAUNCH("engine qkv_post");
+    PackedSeqs wide{};
+    for (int i = 0; i < seqs.n; ++i) {
+        const int n = seqs.len[i];
+        if (n > 8) {
+            wide.row0[wide.n] = seqs.row0[i], wide.len[wide.n] = n, wide.slot[wide.n] = seqs.slot[i], wide.ctx[wide.n] = seqs.ctx[i];
+            ++wide.n;
+            continue;
+        }
+        uint16_t *attn_t = e->attn_t + (size_t)seqs.row0[i] * Hq * D;
+        TL_TRY(engine_paged_attention(e, l, e->q_t + (size_t)seqs.row0[i] * Hq * D, e->block_table + (size_t)seqs.slot[i] * c.max_pages_per_seq, e->scratch_ctx + i,
+                                      attn_t, n, seqs.ctx[i]));
+        hipLaunchKernelGGL(heads_to_rows_kernel, dim3(ceil_div((long)Hq * n * (D / 8), 256)), dim3(256), 0, e->stream, attn_t,
+                           e->attn + (size_t)seqs.row0[i] * Hq * D, Hq, n, D);
+        TL_CHECK_LAUNCH("engine heads to rows");
+    }
+    if (wide.n)
+        TL_TRY(paged_attention_packed(e->q_t, e->layer_k(l), e->layer_v(l), kv8 ? e->layer_ks(l) : nullptr, kv8 ? e->layer_vs(l) : nullptr, e->block_table, e->attn, wide,
+                                      c.page_size, c.max_pages_per_seq, Hq, Hkv, 1.0f / sqrtf((float)D), (float *)e->attn_ws, e->attn_ws_bytes, e->stream));
+    return TL_OK;
 }
 
 static int prefill_impl(tl_engine *e, int slot, const int32_t *tokens, int n, int logits_mode) {
@@ -1901,34 +1948,40 @@ static int prefill_impl(tl_engine *e, int slot, const int32_t *tokens, int n, in
                                   n, c.hidden_size, c.vocab_size, 128, 4, TL_BF16, e->stream));
     const size_t attn_ws_need = tl_paged_attention_workspace_bytes(Hq, n, D, c.page_size, c.max_pages_per_seq, Hq, Hkv, start + n);
     TL_REQUIRE(attn_ws_need <= e->attn_ws_bytes, "engine_prefill: attention workspace too small");
+    PackedSeqs own{};
+    own.n = 1, own.len[0] = n, own.slot[0] = slot, own.ctx[0] = start + n;
     bool x_normed = false;  // the previous layer's w_down reduction left this layer's normalised rows in xn (engine_gemm)
     for (int l = 0; l < c.num_layers; ++l) {
         const tl_layer_weights &w = e->layers[l];
         if (!x_normed) TL_TRY(tl_rms_norm(e->x, w.input_norm_dev, e->xn, n, c.hidden_size, c.rms_norm_eps, TL_BF16, e->stream));
         x_normed = false;
         TL_TRY(engine_gemm(e, w.wqkv, e->xn, e->qkv, n, EPI_STORE, nullptr));
-        QkvPostArgs q{};
-        q.qkv = e->qkv;
-        q.q_norm_w = (const uint16_t *)w.q_norm_dev;
-        q.k_norm_w = (const uint16_t *)w.k_norm_dev;
-        q.q_t = e->q_t;
-        q.key_pages = e->layer_k(l);
-        q.value_pages = e->layer_v(l);
-        q.block_row = block_row;
-        q.T = n;
-        q.start = start;
-        q.page_size = c.page_size;
-        q.max_pages = c.max_pages_per_seq;
-        q.num_heads = Hq;
-        q.num_kv_heads = Hkv;
-        q.eps = c.rms_norm_eps;
-        q.rope_base = c.rope_theta;
-        launch_qkv_post(e, l, q, n);
-        TL_CHECK_LAUNCH("engine qkv_post");
-        TL_TRY(engine_paged_attention(e, l, e->q_t, block_row, e->scratch_ctx, e->attn_t, n, start + n));
-        {
-            const long total = (long)Hq * n * (D / 8);
-            hipLaunchKernelGGL(heads_to_rows_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, e->stream, e->attn_t, e->attn, Hq, n, D);
+        if (n > 8) {
+            TL_TRY(prefill_attention(e, l, own, n));
+        } else {
+            QkvPostArgs q{};
+            q.qkv = e->qkv;
+            q.q_norm_w = (const uint16_t *)w.q_norm_dev;
+            q.k_norm_w = (const uint16_t *)w.k_norm_dev;
+            q.q_t = e->q_t;
+            q.key_pages = e->layer_k(l);
+            q.value_pages = e->layer_v(l);
+            q.block_row = block_row;
+            q.T = n;
+            q.start = start;
+            q.page_size = c.page_size;
+            q.max_pages = c.max_pages_per_seq;
+            q.num_heads = Hq;
+            q.num_kv_heads = Hkv;
+            q.eps = c.rms_norm_eps;
+            q.rope_base = c.rope_theta;
+            launch_qkv_post(e, l, q, n);
+            TL_CHECK_LAUNCH("engine qkv_post");
+            TL_TRY(engine_paged_attention(e, l, e->q_t, block_row, e->scratch_ctx, e->attn_t, n, start + n));
+            {
+                const long total = (long)Hq * n * (D / 8);
+                hipLaunchKernelGGL(heads_to_rows_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, e->stream, e->attn_t, e->attn, Hq, n, D);
+            }
         }
         bool h_normed = false;
         TL_TRY(engine_gemm(e, w.wo, e->attn, e->h, n, EPI_RESIDUAL, e->x, w.post_norm_dev, e->xn, &h_normed));
@@ -1986,8 +2039,8 @@ static int prefill_impl(tl_engine *e, int slot, const int32_t *tokens, int n, in
 }
 
 // Several sequences' chunks in ONE pass of the multi-token path.  The projections (97 % of the prefill FLOPs) run once over the
-// concatenated rows -- a 2,048-row GEMM instead of several 300-row ones -- while RoPE / KV append, the paged FlashAttention
-// and the head transpose stay per sequence (each has its own block-table row, start position and causal mask).
+// concatenated rows -- a 2,048-row GEMM instead of several 300-row ones -- and so do RoPE / KV append and the paged FlashAttention, which look a
+// row's or a block's sequence up (its block-table row, position and causal mask).
 static int prefill_packed_impl(tl_engine *e, int n_seqs, const int *slots, const int32_t *tokens, const int *lens, const int *want_logits) {
     const tl_engine_config &c = e->cfg;
     TL_REQUIRE(e && slots && tokens && lens && want_logits, "engine_prefill_packed: null argument");
@@ -2028,6 +2081,9 @@ static int prefill_packed_impl(tl_engine *e, int n_seqs, const int *slots, const
     pk.clear();
     TL_HIP(hipMemcpyAsync(e->prefill_tokens, tokens, (size_t)total * 4, hipMemcpyHostToDevice, e->stream));
 
+    PackedSeqs seqs{};
+    seqs.n = n_seqs;
+    for (int i = 0; i < n_seqs; ++i) seqs.row0[i] = row0[i], seqs.len[i] = lens[i], seqs.slot[i] = slots[i], seqs.ctx[i] = start[i] + lens[i];
     const int D = c.head_dim, Hq = c.num_heads, Hkv = c.num_kv_heads;
     TL_TRY(tl_quantized_embedding(e->prefill_tokens, 0, e->embed.scales_dev, e->embed.biases_dev, e->embed.weight_dev, e->x,
                                   total, c.hidden_size, c.vocab_size, 128, 4, TL_BF16, e->stream));
@@ -2040,34 +2096,7 @@ static int prefill_packed_impl(tl_engine *e, int n_seqs, const int *slots, const
         if (!x_normed) TL_TRY(tl_rms_norm(e->x, w.input_norm_dev, e->xn, total, c.hidden_size, c.rms_norm_eps, TL_BF16, e->stream));
         x_normed = false;
         TL_TRY(engine_gemm(e, w.wqkv, e->xn, e->qkv, total, EPI_STORE, nullptr));
-        for (int i = 0; i < n_seqs; ++i) {
-            const int n = lens[i];
-            const int32_t *block_row = e->block_table + (size_t)slots[i] * c.max_pages_per_seq;
-            uint16_t *q_t = e->q_t + (size_t)row0[i] * Hq * D;        // this sequence's [Hq][n][D] block
-            uint16_t *attn_t = e->attn_t + (size_t)row0[i] * Hq * D;
-            QkvPostArgs q{};
-            q.qkv = e->qkv + (size_t)row0[i] * (Hq + 2 * Hkv) * D;
-            q.q_norm_w = (const uint16_t *)w.q_norm_dev;
-            q.k_norm_w = (const uint16_t *)w.k_norm_dev;
-            q.q_t = q_t;
-            q.key_pages = e->layer_k(l);
-            q.value_pages = e->layer_v(l);
-            q.block_row = block_row;
-            q.T = n;
-            q.start = start[i];
-            q.page_size = c.page_size;
-            q.max_pages = c.max_pages_per_seq;
-            q.num_heads = Hq;
-            q.num_kv_heads = Hkv;
-            q.eps = c.rms_norm_eps;
-            q.rope_base = c.rope_theta;
-            launch_qkv_post(e, l, q, n);
-            TL_CHECK_LAUNCH("engine qkv_post");
-            TL_TRY(engine_paged_attention(e, l, q_t, block_row, e->scratch_ctx + i, attn_t, n, start[i] + n));
-            const long items = (long)Hq * n * (D / 8);
-            hipLaunchKernelGGL(heads_to_rows_kernel, dim3(ceil_div(items, 256)), dim3(256), 0, e->stream, attn_t,
-                               e->attn + (size_t)row0[i] * Hq * D, Hq, n, D);
-        }
+        TL_TRY(prefill_attention(e, l, seqs, total));
         bool h_normed = false;
         TL_TRY(engine_gemm(e, w.wo, e->attn, e->h, total, EPI_RESIDUAL, e->x, w.post_norm_dev, e->xn, &h_normed));
         if (!h_normed) TL_TRY(tl_rms_norm(e->h, w.post_norm_dev, e->xn, total, c.hidden_size, c.rms_norm_eps, TL_BF16, e->stream));

@@ -1043,26 +1043,41 @@ struct QkvPostArgs {
     float *key_scales, *value_scales;  // KV8: the row scales of FP8 pages (kv8.h); key_pages / value_pages then hold bytes
 };
 
-template <int VD, bool KV8 = false>
-static __global__ __launch_bounds__(256) void qkv_post_kernel(const QkvPostArgs p) {
+// SEQS = PackedSeqs (head dimension 128): the rows of several sequences in one launch; block_row is the block table, T and start come from `seqs`.  The queries
+// of a sequence longer than 8 tokens are left in row order [row][head][128], those of a shorter one as [head][token][128] in its part of q_t.
+struct OneSeq {};
+template <int VD, bool KV8 = false, typename SEQS = OneSeq>
+static __global__ __launch_bounds__(256) void qkv_post_kernel(const QkvPostArgs p, const SEQS seqs) {
     static_assert(!KV8 || VD == 8, "FP8 pages: head dimension 128");
     constexpr int D = 16 * VD;
+    constexpr bool PACKED = !std::is_same<SEQS, OneSeq>::value;
     const int r = blockIdx.x;
+    int T = p.T, start = p.start, t_in = r;  // the row's sequence: its tokens in this pass, the position of the first, the row's place among them
+    const int32_t *block_row = p.block_row;
+    long q_at = 0, q_row = r, q_head = T;    // q_t row of head h: q_at + q_row + h * q_head
+    if constexpr (PACKED) {
+        int i = 0;
+        while (i + 1 < seqs.n && r >= seqs.row0[i + 1]) ++i;
+        T = seqs.len[i], start = seqs.ctx[i] - T, t_in = r - seqs.row0[i];
+        block_row = p.block_row + (long)seqs.slot[i] * p.max_pages;
+        if (T > 8) q_at = (long)r * p.num_heads, q_row = 0, q_head = 1;
+        else q_at = (long)seqs.row0[i] * p.num_heads, q_row = t_in, q_head = T;
+    }
     const int g = threadIdx.x >> 4;
     const int t = threadIdx.x & 15;
     const int Hq = p.num_heads, Hkv = p.num_kv_heads;
-    const int pos = p.start + r;
+    const int pos = start + t_in;
     const uint16_t *row = p.qkv + (long)r * (Hq + 2 * Hkv) * D;
     float cs[VD], sn[VD];
     rope_factors<VD>(t, pos, p.rope_base, cs, sn);
     const int lp = pos / p.page_size;
     const int slot = pos - lp * p.page_size;
-    const int page_id = lp < p.max_pages ? p.block_row[lp] : -1;
+    const int page_id = lp < p.max_pages ? block_row[lp] : -1;
     for (int h = g; h < Hq + 2 * Hkv; h += 16) {
         float v[VD];
         if (h < Hq) {
             head_norm_rope<VD>(row + (long)h * D, p.q_norm_w, t, p.eps, cs, sn, v);
-            store_row<VD>(p.q_t + ((long)h * p.T + r) * D + t * VD, v);
+            store_row<VD>(p.q_t + (q_at + q_row + h * q_head) * D + t * VD, v);
         } else if (h < Hq + Hkv) {
             head_norm_rope<VD>(row + (long)h * D, p.k_norm_w, t, p.eps, cs, sn, v);
             const long prow = ((long)max(page_id, 0) * Hkv + (h - Hq)) * p.page_size + slot;
