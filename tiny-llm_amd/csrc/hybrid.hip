@@ -197,8 +197,8 @@ static int linear_t(const void *A, int lda, const void *W, float *out, int ldc, 
     using S = typename D::storage;
     if (M <= 0 || N <= 0 || batch <= 0) return TL_OK;
     const int vec_ok = (K % 8 == 0) && (lda % 8 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0) && sa % 8 == 0 && sw % 8 == 0;
-    const bool rows = force == 1 || (force == 0 && M <= 8);
-    TL_REQUIRE(!rows || M <= 8, "hybrid linear: the row kernel takes at most 8 rows");
+    const bool rows = force == 1 || (force == 0 && M <= (vec_ok ? 16 : 8));
+    TL_REQUIRE(force != 1 || M <= 8, "hybrid linear: the row kernel takes at most 8 rows");
     if constexpr (sizeof(S) == 2) {
         // large bf16 products: the framework's LDS-DMA 256-wide tile GEMM with its float32 epilogues (gemm8.h); dense operands, whole 64-wide K steps
         const bool big = force == 3 || (force == 0 && M >= 192);
@@ -226,17 +226,30 @@ static int linear_t(const void *A, int lda, const void *W, float *out, int ldc, 
     const BranchTail bt = with_branch ? *branch : BranchTail{};
 #define HY_GEMM(KERN, E) \
     hipLaunchKernelGGL((KERN<D, E>), grid, block, 0, st, (const S *)A, lda, (const S *)W, out, ldc, M, N, K, alpha, bias, vec_ok, sa, sw, sc, nw, nb, nalpha, nout, bt)
-#define HY_GEMM_ROWS(E) \
-    hipLaunchKernelGGL((gemm_rows_kernel<D, E>), grid, block, 0, st, (const S *)A, lda, (const S *)W, out, ldc, M, N, K, alpha, bias, vec_ok, sa, sw, sc, nw, nb, nalpha, nout, sk, bt)
+#define HY_GEMM_ROWS(KERN, E) \
+    hipLaunchKernelGGL(KERN, grid, block, 0, st, (const S *)A, lda, (const S *)W, out, ldc, M, N, K, alpha, bias, ks, sa, sw, sc, nw, nb, nalpha, nout, sk, bt)
+#define HY_GEMM_ROWS_C(E)                                                    \
+    do {                                                                     \
+        if (!blocked) HY_GEMM_ROWS((gemm_rows_any_kernel<D, E>), E);         \
+        else if (M <= 4) HY_GEMM_ROWS((gemm_rows_kernel<D, E, 4>), E);       \
+        else if (M <= 8) HY_GEMM_ROWS((gemm_rows_kernel<D, E, 8>), E);       \
+        else HY_GEMM_ROWS((gemm_rows_kernel<D, E, 16>), E);                  \
+    } while (0)
     if (rows) {
-        dim3 grid((N + 3) / 4, batch), block(256);
+        // columns a matrix instruction holds, and the waves that split a column block's K: the fewest that give every CU two workgroups (at least a chunk each)
+        const bool blocked = vec_ok && (sizeof(S) == 2 || M > 4 || K >= 2048);
+        const int C = M <= 4 ? 4 : (M <= 8 ? 8 : 16), blocks = (N + C - 1) / C, chunk = 16 / C * 64 / (int)sizeof(S);
+        int ks = 1;
+        while (ks < 4 && (long)blocks * batch * ks / 4 < 2 * qmm3_num_cus() && 8 * ks * chunk <= K) ks *= 2;
+        if (!blocked) ks = vec_ok;
+        dim3 grid(blocked ? (blocks * ks + 3) / 4 : (N + 3) / 4, batch), block(256);
         const SegSkip sk = skip ? *skip : SegSkip{};
-        if (with_branch) HY_GEMM_ROWS(5);
-        else if (epi == 0) HY_GEMM_ROWS(0);
-        else if (epi == 1) HY_GEMM_ROWS(1);
-        else if (epi == 2) HY_GEMM_ROWS(2);
-        else if (!with_tail) HY_GEMM_ROWS(3);
-        else HY_GEMM_ROWS(4);
+        if (with_branch) HY_GEMM_ROWS_C(5);
+        else if (epi == 0) HY_GEMM_ROWS_C(0);
+        else if (epi == 1) HY_GEMM_ROWS_C(1);
+        else if (epi == 2) HY_GEMM_ROWS_C(2);
+        else if (!with_tail) HY_GEMM_ROWS_C(3);
+        else HY_GEMM_ROWS_C(4);
     } else {
         dim3 grid(((M + 63) / 64) * ((N + 63) / 64), batch), block(256);
         if (with_branch) HY_GEMM(gemm_tile_kernel, 5);
@@ -248,6 +261,7 @@ static int linear_t(const void *A, int lda, const void *W, float *out, int ldc, 
     }
 #undef HY_GEMM
 #undef HY_GEMM_ROWS
+#undef HY_GEMM_ROWS_C
     if (with_tail) tail->done = true;
     if (branch_done) *branch_done = with_branch;
     TL_CHECK_LAUNCH("hybrid linear");

@@ -5,6 +5,8 @@
 // sequence list) and row_pos (position in its sequence).  Per sequence: seq_row0 (first row; seq_row0[n] = rows),
 // seq_slot (state slot = block-table row).
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace tl {
@@ -155,6 +157,23 @@ __device__ __forceinline__ void branch_tail(const BranchTail &t, size_t i, int n
     if (t.h) reinterpret_cast<typename D::storage *>(t.h)[i] = D::from_float(tanhf(t.nalpha * v) * t.nw[n] + t.nb[n]);
 }
 
+// What an output element of a product becomes (EPI as below).
+template <typename D, int EPI>
+__device__ __forceinline__ void product_out(float *out, int ldc, int N, int m, int n, float v, float alpha, const float *bias, const float *nw, const float *nb,
+                                            float nalpha, typename D::storage *nout, const BranchTail &tail) {
+    float *o = out + (size_t)m * ldc + n;
+    if constexpr (EPI == 0) *o = v;
+    else if constexpr (EPI == 1) *o += alpha * v;
+    else if constexpr (EPI == 2) *o = v + bias[n];
+    else if constexpr (EPI == 3) *o += alpha * bias[n] * v;
+    else if constexpr (EPI == 5) branch_tail<D>(tail, (size_t)m * N + n, n, v);
+    else {
+        const float xn = *o + alpha * bias[n] * v;
+        *o = xn;
+        nout[(size_t)m * N + n] = D::from_float(tanhf(nalpha * xn) * nw[n] + nb[n]);
+    }
+}
+
 // ---- tile matrix product: out[M, N] (+)= A[M, K] . W[N, K]^T, float32 accumulation on the matrix cores ------------
 // 64 x 64 output tile per 256-thread workgroup, 4 waves of 32 x 32 (2 x 2 MFMA 16x16 tiles), K in steps of 32 through LDS.
 // bf16: v_mfma_f32_16x16x32_bf16; fp32: v_mfma_f32_16x16x4_f32 (full fp32 products).  Any M, N, K: edges are zero-filled in LDS.
@@ -262,18 +281,7 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(const typename D::storag
             for (int r = 0; r < 4; ++r) {
                 const int gm = m0 + wm * 32 + i * 16 + (lane >> 4) * 4 + r, gn = n0 + wn * 32 + j * 16 + (lane & 15);
                 if (gm < M && gn < N) {
-                    float *o = out + (size_t)gm * ldc + gn;
-                    const float v = acc[i][j][r];
-                    if constexpr (EPI == 0) *o = v;
-                    else if constexpr (EPI == 1) *o += alpha * v;
-                    else if constexpr (EPI == 2) *o = v + bias[gn];
-                    else if constexpr (EPI == 3) *o += alpha * bias[gn] * v;
-                    else if constexpr (EPI == 5) branch_tail<D>(tail, (size_t)gm * N + gn, gn, v);
-                    else {
-                        const float xn = *o + alpha * bias[gn] * v;
-                        *o = xn;
-                        nout[(size_t)gm * N + gn] = D::from_float(tanhf(nalpha * xn) * nw[gn] + nb[gn]);
-                    }
+                    product_out<D, EPI>(out, ldc, N, gm, gn, acc[i][j][r], alpha, bias, nw, nb, nalpha, nout, tail);
                 }
             }
 }
@@ -287,13 +295,105 @@ struct SegSkip {
     int lead = 0, len = 1, period = 1, limit = 0, on_k = 0;
 };
 
-// ---- row matrix product for a few rows (decode): each wave owns one output column and streams its weight row once ----
-// M <= 8.  Lanes stride over K, 8 elements at a time where the layout allows 16-byte loads.
+// ---- matrix product for up to 16 rows (decode): bound by streaming W once, i.e. by how many of its bytes are in flight ----
+// A 16 x 16 matrix instruction holds C = 4, 8 or 16 columns of W in S = 16 / C phases of K: its row c + C s is column c over the s-th piece of the chunk, its
+// column m + C s row m of A over the same piece, so the blocks with equal phases on its result's diagonal are partial sums of out[m][c] (M <= C).  Lane l
+// serves row AND column l % 16: one k for both of its 16-byte loads.  A wave requests 8 chunks (8 KB of W) before it multiplies; `ks` waves share a column
+// block and split its chunks between them (interleaved), 4 / ks column blocks a workgroup: few columns (1,024 of K = 4,096: 256 workgroups of 4 columns, 33 KB
+// each) keep every CU's loads in flight as many do.  Measured against one wave per column with the next load behind the last one's multiply-adds (launch to
+// launch): that product (8.4 MB, 4 rows) 12.5 -> 4.8 us, 8,192 deep for 2,048 columns (34 MB, 1 row) 16.1 -> 8.5, 32,768 columns of K = 1,024 (67 MB, 4 rows)
+// 25.6 -> 17.4; 9 .. 16 rows were 64 x 64 tiles: 2,048 columns of K = 2,048, 16 rows 50 -> 7 us.  Error against 64 bits as before (8e-8).
+// K % 8 == 0, 16-byte aligned rows; other layouts: gemm_rows_any_kernel.
+template <typename D, int EPI, int C>
+__global__ __launch_bounds__(256) void gemm_rows_kernel(const typename D::storage *A, int lda, const typename D::storage *W, float *out, int ldc, int M, int N, int K,
+                                                        float alpha, const float *bias, int ks, long sa, long sw, long sc, const float *nw, const float *nb,
+                                                        float nalpha, typename D::storage *nout, SegSkip skip, BranchTail tail) {
+    using S = typename D::storage;
+    constexpr int PH = 16 / C, VEC = 16 / (int)sizeof(S), PIECE = 4 * VEC, CH = PH * PIECE;
+    __shared__ f32x4 red[4 * 64];
+    A += (size_t)blockIdx.y * sa, W += (size_t)blockIdx.y * sw, out += (size_t)blockIdx.y * sc;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, lr = lane & 15;
+    const int groups = 4 / ks, n0 = ((int)blockIdx.x * groups + wave / ks) * C, part = wave % ks;
+    const int c = lr % C, ph = lr / C;
+    const unsigned long long need = skip.mask ? *skip.mask : ~0ull;
+    bool wanted = n0 < N;
+    if (skip.mask && !skip.on_k) {
+        const int n = n0 + c, at = n % skip.period;
+        wanted = __any(n < N && (n >= skip.limit || at < skip.lead || ((need >> ((at - skip.lead) / skip.len)) & 1ull)));
+    }
+    const bool k_skip = skip.mask && skip.on_k;
+    const S *wrow = W + (size_t)min(n0 + c, N - 1) * K, *arow = A + (size_t)min(c, M - 1) * lda;  // (columns behind N and rows behind M are not written)
+    f32x4 acc[8];  // (a sum per chunk in flight: short sums, added pairwise behind the loop)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto batch = [&](auto count, int k0) __attribute__((always_inline)) {
+        constexpr int U = decltype(count)::value;
+        u32x4 wv[U], av[U];
+        bool ok[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u * ks * CH + PIECE * ph + VEC * g;
+            ok[u] = k < K;
+            if (k_skip && ok[u] && k >= skip.lead) ok[u] = (need >> ((k - skip.lead) / skip.len)) & 1ull;
+            const int at = ok[u] ? k : 0;
+            wv[u] = *reinterpret_cast<const u32x4 *>(wrow + at);
+            av[u] = *reinterpret_cast<const u32x4 *>(arow + at);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (!ok[u]) wv[u] = av[u] = u32x4{0u, 0u, 0u, 0u};
+            if constexpr (sizeof(S) == 2) {
+                acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wv[u]), __builtin_bit_cast(bf16x8_t, av[u]), acc[u], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int to = U == 8 ? u : (U * e + u) % 8;
+                    acc[to] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(wv[u][e]), __uint_as_float(av[u][e]), acc[to], 0, 0, 0);
+                }
+            }
+        }
+    };
+    if (wanted) {
+        int k0 = part * CH, left = ((K + CH - 1) / CH - part + ks - 1) / ks;  // the wave's chunks
+        for (; left >= 8; left -= 8, k0 += 8 * ks * CH) batch(std::integral_constant<int, 8>{}, k0);
+        if (left & 4) batch(std::integral_constant<int, 4>{}, k0), k0 += 4 * ks * CH;
+        if (left & 2) batch(std::integral_constant<int, 2>{}, k0), k0 += 2 * ks * CH;
+        if (left & 1) batch(std::integral_constant<int, 1>{}, k0);
+    }
+    // result: lane holds rows 4 g + e (column (4 g + e) % C of phase (4 g + e) / C) of its own column (row m of phase ph)
+    red[wave * 64 + lane] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+    __syncthreads();
+    const float *rf = reinterpret_cast<const float *>(red);
+    for (int i = threadIdx.x; i < groups * C * C; i += 256) {
+        const int grp = i / (C * C), m = (i / C) % C, col = i % C, n = ((int)blockIdx.x * groups + grp) * C + col;
+        if (m >= M || n >= N) continue;
+        if (skip.mask && !skip.on_k) {  // a block without a needed column was not computed; its consumers do not read it
+            const int at = n % skip.period;
+            if (!(n >= skip.limit || at < skip.lead || ((need >> ((at - skip.lead) / skip.len)) & 1ull))) continue;
+        }
+        auto share = [&](int p) {  // a wave's sum over the phases
+            float q[PH];
+#pragma unroll
+            for (int s = 0; s < PH; ++s) {
+                const int row = col + C * s, from = 16 * (row / 4) + m + C * s;
+                q[s] = rf[((grp * ks + p) * 64 + from) * 4 + row % 4];
+            }
+            if constexpr (PH == 4) return (q[0] + q[1]) + (q[2] + q[3]);
+            else if constexpr (PH == 2) return q[0] + q[1];
+            else return q[0];
+        };
+        const float v = ks == 4 ? (share(0) + share(1)) + (share(2) + share(3)) : (ks == 2 ? share(0) + share(1) : share(0));
+        product_out<D, EPI>(out, ldc, N, m, n, v, alpha, bias, nw, nb, nalpha, nout, tail);
+    }
+}
+
+// the same for up to 8 rows of any K, alignment and strides: a wave per output column, element by element.  vec (float32 rows that 16-byte loads fit): 8 elements a
+// lane at a time; a matrix instruction of float32 takes 8 times a bf16 one's time, so this stays the faster form for short K and few rows (7,184 columns of
+// K = 1,024, 1 row: 7.8 us against 10.0).
 template <typename D, int EPI>
-__global__ __launch_bounds__(256) void gemm_rows_kernel(const typename D::storage *A, int lda, const typename D::storage *W, float *out,
-                                                        int ldc, int M, int N, int K, float alpha, const float *bias, int vec_ok, long sa, long sw,
-                                                        long sc, const float *nw, const float *nb, float nalpha, typename D::storage *nout,
-                                                        SegSkip skip, BranchTail tail) {
+__global__ __launch_bounds__(256) void gemm_rows_any_kernel(const typename D::storage *A, int lda, const typename D::storage *W, float *out, int ldc, int M, int N, int K,
+                                                            float alpha, const float *bias, int vec, long sa, long sw, long sc, const float *nw, const float *nb,
+                                                            float nalpha, typename D::storage *nout, SegSkip skip, BranchTail tail) {
     using S = typename D::storage;
     A += (size_t)blockIdx.y * sa, W += (size_t)blockIdx.y * sw, out += (size_t)blockIdx.y * sc;
     const int lane = threadIdx.x & 63;
@@ -309,21 +409,12 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const typename D::storag
 #pragma unroll
     for (int m = 0; m < 8; ++m) acc[m] = 0.f;
     const S *wrow = W + (size_t)n * K;
-    if (vec_ok) {
-        for (int k = lane * 8; k + 8 <= K; k += 64 * 8) {
+    if (sizeof(S) == 4 && vec) {
+        for (int k = lane * 8; k < K; k += 64 * 8) {  // (K and the segments are multiples of 8)
             if (k_skip && k >= skip.lead && !((need >> ((k - skip.lead) / skip.len)) & 1ull)) continue;
             float wf[8];
-            if constexpr (sizeof(S) == 2) {
-                u32x4 u = *reinterpret_cast<const u32x4 *>(wrow + k);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    wf[2 * i] = __uint_as_float(u[i] << 16);
-                    wf[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) wf[i] = D::to_float(wrow[k + i]);
-            }
+            for (int i = 0; i < 8; ++i) wf[i] = D::to_float(wrow[k + i]);
 #pragma unroll
             for (int m = 0; m < 8; ++m) {
                 if (m < M) {
@@ -333,14 +424,9 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const typename D::storag
                 }
             }
         }
-        for (int k = (K / 8) * 8 + lane; k < K; k += 64) {
-            const float wf = D::to_float(wrow[k]);
-#pragma unroll
-            for (int m = 0; m < 8; ++m)
-                if (m < M) acc[m] += wf * D::to_float(A[(size_t)m * lda + k]);
-        }
     } else {
         for (int k = lane; k < K; k += 64) {
+            if (k_skip && k >= skip.lead && !((need >> ((k - skip.lead) / skip.len)) & 1ull)) continue;
             const float wf = D::to_float(wrow[k]);
 #pragma unroll
             for (int m = 0; m < 8; ++m)
@@ -351,19 +437,7 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const typename D::storag
     for (int m = 0; m < 8; ++m) {
         if (m < M) {  // M is uniform over the grid
             const float v = wave_sum(acc[m]);
-            if (lane == 0) {
-                float *o = out + (size_t)m * ldc + n;
-                if constexpr (EPI == 0) *o = v;
-                else if constexpr (EPI == 1) *o += alpha * v;
-                else if constexpr (EPI == 2) *o = v + bias[n];
-                else if constexpr (EPI == 3) *o += alpha * bias[n] * v;
-                else if constexpr (EPI == 5) branch_tail<D>(tail, (size_t)m * N + n, n, v);
-                else {
-                    const float xn = *o + alpha * bias[n] * v;
-                    *o = xn;
-                    nout[(size_t)m * N + n] = D::from_float(tanhf(nalpha * xn) * nw[n] + nb[n]);
-                }
-            }
+            if (lane == 0) product_out<D, EPI>(out, ldc, N, m, n, v, alpha, bias, nw, nb, nalpha, nout, tail);
         }
     }
 }
