@@ -237,7 +237,7 @@ static int linear_t(const void *A, int lda, const void *W, float *out, int ldc, 
     } while (0)
     if (rows) {
         // columns a matrix instruction holds, and the waves that split a column block's K: the fewest that give every CU two workgroups (at least a chunk each)
-        const bool blocked = vec_ok && (sizeof(S) == 2 || M > 4 || K >= 2048);
+        const bool blocked = vec_ok && (sizeof(S) == 2 || M > 4);
         const int C = M <= 4 ? 4 : (M <= 8 ? 8 : 16), blocks = (N + C - 1) / C, chunk = 16 / C * 64 / (int)sizeof(S);
         int ks = 1;
         while (ks < 4 && (long)blocks * batch * ks / 4 < 2 * qmm3_num_cus() && 8 * ks * chunk <= K) ks *= 2;
@@ -356,15 +356,16 @@ struct StepShape {
     int n_splits = 1, keys_per_split = 1 << 30;  // attention: the key range of a row split over workgroups (decode steps over long contexts)
 };
 
-// how a step's attention splits the keys: only steps of single tokens, from 256 keys on; one 64-key tile per split, doubled until at most 64
-// splits (a decode step is a few rows: its time is the chain of tiles a workgroup walks, so the chain is kept short and the chip full)
+// how a step's attention splits the keys: only steps of single tokens; one 64-key tile per split, doubled until at most 64 splits (a decode step is a few rows:
+// its time is the chain of tiles a workgroup walks, so the chain is kept short and the chip full: 4 sequences of 200 .. 248 keys, 8 heads: 18 us in one walk,
+// 7 + 5 for the merge in four splits).  At least 4 splits: the first 256 tokens of a context share one captured step (up to 64 keys: 11 us in one walk as it was).
 static void plan_splits(StepShape &sh, int ctx_bound) {
     sh.n_splits = 1;
     sh.keys_per_split = 1 << 30;
-    if (sh.max_len != 1 || ctx_bound <= 256) return;
+    if (sh.max_len != 1) return;
     int kps = 64;
     while ((ctx_bound + kps - 1) / kps > 64) kps *= 2;
-    int n = 1;
+    int n = 4;
     while (n * kps < ctx_bound) n *= 2;
     sh.n_splits = n;
     sh.keys_per_split = kps;
@@ -424,7 +425,7 @@ static int launch_attn_tile(tl_hybrid *e, const tl_hybrid_layer &L, const void *
                        x.softcap, x.slopes, x.sinks, x.out_scale, x.keep_first);
     TL_CHECK_LAUNCH("hybrid attention tile");
     if (sh.n_splits > 1) {
-        hipLaunchKernelGGL((attn_merge_kernel<D>), dim3(sh.rows, L.heads), dim3(256), 0, e->stream, e->part_acc, e->part_ml, sh.n_splits, L.heads, L.vdim, gate,
+        hipLaunchKernelGGL((L.vdim % 4 == 0 ? attn_merge_kernel<D, 4> : attn_merge_kernel<D, 1>), dim3(sh.rows, L.heads), dim3(256), 0, e->stream, e->part_acc, e->part_ml, sh.n_splits, L.heads, L.vdim, gate,
                            ldg, (S *)out, ldo, x.gate_per_head, x.out32, x.out_scale);
         TL_CHECK_LAUNCH("hybrid attention merge");
     }
@@ -454,7 +455,7 @@ static int launch_attn_pair_tile(tl_hybrid *e, const tl_hybrid_layer &L, const v
                        (uint16_t *)out, ldo, e->part_acc, e->part_ml, x.window, x.vshare, x.gate_per_head, x.out32, x.softcap, x.slopes, x.sinks, x.out_scale, x.keep_first);
     TL_CHECK_LAUNCH("hybrid attention tile (bfloat16 pairs)");
     if (sh.n_splits > 1) {
-        hipLaunchKernelGGL((attn_merge_kernel<BF16>), dim3(sh.rows, L.heads), dim3(256), 0, e->stream, e->part_acc, e->part_ml, sh.n_splits, L.heads, L.vdim, gate, ldg,
+        hipLaunchKernelGGL((L.vdim % 4 == 0 ? attn_merge_kernel<BF16, 4> : attn_merge_kernel<BF16, 1>), dim3(sh.rows, L.heads), dim3(256), 0, e->stream, e->part_acc, e->part_ml, sh.n_splits, L.heads, L.vdim, gate, ldg,
                            (uint16_t *)out, ldo, x.gate_per_head, x.out32, x.out_scale);
         TL_CHECK_LAUNCH("hybrid attention merge");
     }
@@ -514,7 +515,7 @@ static int launch_latent_tile(tl_hybrid *e, const tl_hybrid_layer &L, const void
                        sh.n_splits, (uint16_t *)out, L.heads * L.kv_rank, e->part_acc, e->part_ml);
     TL_CHECK_LAUNCH("hybrid latent attention tile");
     if (sh.n_splits > 1) {
-        hipLaunchKernelGGL((attn_merge_kernel<BF16>), dim3(sh.rows, L.heads), dim3(256), 0, e->stream, e->part_acc, e->part_ml, sh.n_splits, L.heads, L.kv_rank,
+        hipLaunchKernelGGL((L.kv_rank % 4 == 0 ? attn_merge_kernel<BF16, 4> : attn_merge_kernel<BF16, 1>), dim3(sh.rows, L.heads), dim3(256), 0, e->stream, e->part_acc, e->part_ml, sh.n_splits, L.heads, L.kv_rank,
                            (const float *)nullptr, 0, (uint16_t *)out, L.heads * L.kv_rank, 0, (float *)nullptr, 1.f);
         TL_CHECK_LAUNCH("hybrid attention merge");
     }
@@ -566,7 +567,7 @@ static int launch_attn_talk_tile(tl_hybrid *e, const tl_hybrid_layer &L, const v
                        sh.keys_per_split, sh.n_splits, gate, ldg, (S *)out, ldo, e->part_acc, e->part_ml, page_shift, vec_ok);
     TL_CHECK_LAUNCH("hybrid attention tile (mixed heads)");
     if (sh.n_splits > 1) {
-        hipLaunchKernelGGL((attn_merge_kernel<D>), dim3(sh.rows, L.heads), dim3(256), 0, e->stream, e->part_acc, e->part_ml, sh.n_splits, L.heads, L.vdim, gate,
+        hipLaunchKernelGGL((L.vdim % 4 == 0 ? attn_merge_kernel<D, 4> : attn_merge_kernel<D, 1>), dim3(sh.rows, L.heads), dim3(256), 0, e->stream, e->part_acc, e->part_ml, sh.n_splits, L.heads, L.vdim, gate,
                            ldg, (S *)out, ldo, 0, (float *)nullptr, 1.f);
         TL_CHECK_LAUNCH("hybrid attention merge");
     }

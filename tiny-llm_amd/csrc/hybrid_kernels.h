@@ -642,6 +642,14 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(const float *qbuf, const
     const int nb = WSPLIT ? wave : 0;
     const bool row_ok = t0 + tl < len && hb < HG;
     const int trow = r0 + t0 + tl, head = kvh * HG + hb, qpos = pos0 + t0 + tl;
+    if (n_splits > 1 && split > 0 && k_begin >= k_end) {  // a split without keys (the sink is split 0's): the merge reads nothing but its maximum
+        if (row_ok && g4 == 0 && (!WSPLIT || wave == 0)) {
+            const size_t pi = ((size_t)trow * H + head) * n_splits + split;
+            part_ml[2 * pi] = -INFINITY;
+            part_ml[2 * pi + 1] = 0.f;
+        }
+        return;
+    }
     const bool owns_sink = sink && split == 0 && (!WSPLIT || wave == 0);
     const float slope = (slopes && row_ok) ? slopes[head] : 0.f, inv_cap = softcap > 0.f ? 1.f / softcap : 0.f;
     float m_run = owns_sink ? (sinks && row_ok ? sinks[head] : 0.f) : -INFINITY, l_run = owns_sink ? 1.f : 0.f;
@@ -651,21 +659,23 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(const float *qbuf, const
     if (k_begin < k_end) {
         float qf[KB16 ? 1 : DK4];       // float32 pages: B operand of the 16x16x4 product, scale folded in
         u32x4 qb[KB16 ? DK4 / 8 : 1];   // bfloat16 pages: B operand of the 16x16x32 product, 8 consecutive k per lane
+        const float *qrow = qbuf + ((size_t)(row_ok ? trow : r0) * H + (row_ok ? head : 0)) * dim;  // (loads from clamped places: none stands behind a branch, see below)
         if constexpr (KB16) {
 #pragma unroll
             for (int ks8 = 0; ks8 < DK4 / 8; ++ks8) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int d = 32 * ks8 + 8 * g4 + 2 * e;
-                    const float *qrow = qbuf + ((size_t)trow * H + head) * dim;
-                    qb[ks8][e] = BF16::pack2((row_ok && d < dim) ? qrow[d] : 0.f, (row_ok && d + 1 < dim) ? qrow[d + 1] : 0.f);
+                    const float q0 = qrow[min(d, dim - 1)], q1 = qrow[min(d + 1, dim - 1)];
+                    qb[ks8][e] = BF16::pack2((row_ok && d < dim) ? q0 : 0.f, (row_ok && d + 1 < dim) ? q1 : 0.f);
                 }
             }
         } else {
 #pragma unroll
             for (int kk = 0; kk < DK4; ++kk) {
                 const int d = 4 * kk + g4;
-                qf[kk] = (row_ok && d < dim) ? qbuf[((size_t)trow * H + head) * dim + d] * scale : 0.f;
+                const float q0 = qrow[min(d, dim - 1)];
+                qf[kk] = (row_ok && d < dim) ? q0 * scale : 0.f;
             }
         }
         // Staging: a tile is 64 (ck + cv) chunks of 8 elements; thread t owns chunks t, t + 256, ... -- the same (key, column) places in every
@@ -682,7 +692,29 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(const float *qbuf, const
             else place[it] = ((q - 64 * ck) / cv) | (((q - 64 * ck) % cv) << 8) | (1 << 24);
         }
         S raw[NIT][8];
+        // vec_ok (widths are multiples of 8: a chunk is whole or absent): every load is issued, rows past the last key and columns past the width from a clamped
+        // place and zeroed on their way into LDS -- a branch around a load makes the compiler wait for it, and for all before it, where the branch ends.
         auto load_tile = [&](int kb) __attribute__((always_inline)) {
+            if (vec_ok) {
+                size_t row[NIT];
+#pragma unroll
+                for (int it = 0; it < NIT; ++it) {
+                    const int pl = max(place[it], 0), jc = min(kb + (pl & 255), k_end - 1), j = jc + (jc >= keep_first ? gap : 0);
+                    const int pg = page_shift >= 0 ? (j >> page_shift) : (j / page_size);
+                    const bool is_v = (pl >> 24) & 1;
+                    row[it] = ((size_t)bt[pg] * (is_v ? Gv : G) + (is_v ? kvh_v : kvh)) * page_size + (j - pg * page_size);
+                }
+#pragma unroll
+                for (int it = 0; it < NIT; ++it) {
+                    const int pl = max(place[it], 0), c8 = 8 * ((pl >> 8) & 0xffff);
+                    const bool is_v = (pl >> 24) & 1;
+                    const int wd = is_v ? vdim : dim;  // v_row: the width of a row of vpool (vdim, or the key row's when the values are its leading columns)
+                    const S *src = (is_v ? vpool + row[it] * v_row : kpool + row[it] * dim) + (c8 < wd ? c8 : 0);
+                    *reinterpret_cast<u32x4 *>(raw[it]) = *reinterpret_cast<const u32x4 *>(src);
+                    if constexpr (sizeof(S) == 4) *reinterpret_cast<u32x4 *>(raw[it] + 4) = *reinterpret_cast<const u32x4 *>(src + 4);
+                }
+                return;
+            }
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
                 const int pl = place[it], jc = kb + (pl & 255), j = jc + (jc >= keep_first ? gap : 0), c8 = 8 * ((pl >> 8) & 0xffff);
@@ -691,28 +723,23 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(const float *qbuf, const
                 for (int e = 0; e < 8; ++e) raw[it][e] = (S)0;
                 if (pl >= 0 && jc < k_end && c8 < (is_v ? vdim : dim)) {
                     const int pg = page_shift >= 0 ? (j >> page_shift) : (j / page_size), in_pg = j - pg * page_size;
-                    const int wd = is_v ? vdim : dim;  // v_row: the width of a row of vpool (vdim, or the key row's when the values are its leading columns)
+                    const int wd = is_v ? vdim : dim;
                     const S *src = (is_v ? vpool + (((size_t)bt[pg] * Gv + kvh_v) * page_size + in_pg) * v_row
                                          : kpool + (((size_t)bt[pg] * G + kvh) * page_size + in_pg) * dim) + c8;
-                    if (vec_ok) {  // (widths are multiples of 8: a chunk is whole or absent)
-                        if constexpr (sizeof(S) == 2) *reinterpret_cast<u32x4 *>(raw[it]) = *reinterpret_cast<const u32x4 *>(src);
-                        else {
-                            *reinterpret_cast<u32x4 *>(raw[it]) = *reinterpret_cast<const u32x4 *>(src);
-                            *reinterpret_cast<u32x4 *>(raw[it] + 4) = *reinterpret_cast<const u32x4 *>(src + 4);
-                        }
-                    } else {
 #pragma unroll
-                        for (int e = 0; e < 8; ++e)
-                            if (c8 + e < wd) raw[it][e] = src[e];
-                    }
+                    for (int e = 0; e < 8; ++e)
+                        if (c8 + e < wd) raw[it][e] = src[e];
                 }
             }
         };
-        auto store_tile = [&]() __attribute__((always_inline)) {
+        auto store_tile = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
                 const int pl = place[it];
                 if (pl < 0) continue;
+                const bool live = kb + (pl & 255) < k_end && 8 * ((pl >> 8) & 0xffff) < (((pl >> 24) & 1) ? vdim : dim);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) raw[it][e] = live ? raw[it][e] : (S)0;
                 if constexpr (KB16) {
                     if (!((pl >> 24) & 1)) {  // a K chunk: 8 bfloat16 as they are
                         *reinterpret_cast<u32x4 *>(reinterpret_cast<uint16_t *>(Ks) + (pl & 255) * (2 * DKP) + 8 * ((pl >> 8) & 0xffff)) =
@@ -734,9 +761,9 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(const float *qbuf, const
         load_tile(k_begin);
         for (int kb = k_begin; kb < k_end; kb += 64) {
             __syncthreads();  // every wave is done with the previous tile
-            store_tile();
+            store_tile(kb);
             __syncthreads();
-            if (kb + 64 < k_end) load_tile(kb + 64);
+            load_tile(kb + 64);
             f32x4 sc[NN];
             float m_tile = -INFINITY;
 #pragma unroll
@@ -864,35 +891,54 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(const float *qbuf, const
 }
 
 // the splits of a row's key range put together: one workgroup per (row, query head), n_splits <= 64.  Lane s of every wave owns split s for the maximum, the
-// sum and the weights exp(m_s - M); then the lanes turn to the value columns, wave w walks the splits w, w + 4, ... with those weights, and the four sums meet in LDS.
-template <typename D>
+// sum and the weights exp(m_s - M); then a lane takes four value columns (1 where vdim is no multiple of 4), wave w walks the splits w, w + 4, ... with those weights, and
+// the four sums meet in LDS.  Splits behind the last one with keys are not read (their tiles leave nothing but m = -inf).
+template <typename D, int VEC>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const float *part_acc, const float *part_ml, int n_splits, int H, int vdim, const float *gate,
                                                          int ldg, typename D::storage *out, int ldo, int gate_per_head, float *out32, float out_scale) {
-    __shared__ float ws[64], sums[4][64];
+    __shared__ float ws[64];
+    __shared__ __attribute__((aligned(16))) float sums[4][64 * VEC];
     const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const size_t p0 = ((size_t)t * H + h) * n_splits;
     const float m = lane < n_splits ? part_ml[2 * (p0 + lane)] : -INFINITY;
     const float l = lane < n_splits ? part_ml[2 * (p0 + lane) + 1] : 0.f;
+    const unsigned long long alive = __ballot(m != -INFINITY);
+    const int live = alive ? 64 - __clzll((long long)alive) : 0;
     const float M = wave_max(m);
     const float w = (m == -INFINITY) ? 0.f : expf(m - M);
     const float L = wave_sum(l * w);
     if (wave == 0) ws[lane] = w;
     const float invl = L > 0.f ? out_scale / L : 0.f;
-    for (int c0 = 0; c0 < vdim; c0 += 64) {
-        const int c = c0 + lane;
+    for (int c0 = 0; c0 < vdim; c0 += 64 * VEC) {
+        const int c = c0 + VEC * lane;
         __syncthreads();
-        float acc = 0.f;
+        float acc[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
         if (c < vdim) {
-#pragma unroll 8
-            for (int s = wave; s < n_splits; s += 4) acc += part_acc[(p0 + s) * vdim + c] * ws[s];
+#pragma unroll 4
+            for (int s = wave; s < live; s += 4) {
+                const float *src = part_acc + (p0 + s) * vdim + c;
+                if constexpr (VEC == 4) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(src);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[e] += v[e] * ws[s];
+                } else {
+                    acc[0] += src[0] * ws[s];
+                }
+            }
         }
-        sums[wave][lane] = acc;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) sums[wave][VEC * lane + e] = acc[e];
         __syncthreads();
-        if (wave != 0 || c >= vdim) continue;
-        float val = ((sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane])) * invl;
-        if (gate) val *= sigmoid_f(gate[(size_t)t * ldg + (gate_per_head ? (size_t)h : (size_t)h * vdim + c)]);
-        if (out32) out32[((size_t)t * H + h) * vdim + c] = val;
-        else out[(size_t)t * ldo + (size_t)h * vdim + c] = D::from_float(val);
+        for (int i = threadIdx.x; i < 64 * VEC; i += 256) {
+            const int cc = c0 + i;
+            if (cc >= vdim) continue;
+            float val = ((sums[0][i] + sums[1][i]) + (sums[2][i] + sums[3][i])) * invl;
+            if (gate) val *= sigmoid_f(gate[(size_t)t * ldg + (gate_per_head ? (size_t)h : (size_t)h * vdim + cc)]);
+            if (out32) out32[((size_t)t * H + h) * vdim + cc] = val;
+            else out[(size_t)t * ldo + (size_t)h * vdim + cc] = D::from_float(val);
+        }
     }
 }
 
@@ -935,6 +981,14 @@ __global__ __launch_bounds__(256) void attn_pair_tile_kernel(const float *qbuf, 
     const int nb = WSPLIT ? wave : 0;
     const bool row_ok = t0 + tl < len && hb < HG;
     const int trow = r0 + t0 + tl, qpos = pos0 + t0 + tl, head = kvh * HG + hb;
+    if (n_splits > 1 && split > 0 && k_begin >= k_end) {  // a split without keys (the sink is split 0's): the merge reads nothing but its maximum
+        if (row_ok && g4 == 0 && (!WSPLIT || wave == 0)) {
+            const size_t pi = ((size_t)trow * H + head) * n_splits + split;
+            part_ml[2 * pi] = -INFINITY;
+            part_ml[2 * pi + 1] = 0.f;
+        }
+        return;
+    }
     const bool owns_sink = sink && split == 0 && (!WSPLIT || wave == 0);
     const float slope = (slopes && row_ok) ? slopes[head] : 0.f, inv_cap = softcap > 0.f ? 1.f / softcap : 0.f;
     float m_run = owns_sink ? (sinks && row_ok ? sinks[head] : 0.f) : -INFINITY, l_run = owns_sink ? 1.f : 0.f;
@@ -942,32 +996,45 @@ __global__ __launch_bounds__(256) void attn_pair_tile_kernel(const float *qbuf, 
 #pragma unroll
     for (int v = 0; v < VT; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (k_begin < k_end) {
+        // A tile travels through registers while the one before it is worked on, the ids of its pages a tile ahead of that.  No load stands behind a branch --
+        // rows past the last key repeat it and are zeroed on their way into LDS -- because the compiler waits for every outstanding load where a branch around
+        // one ends: that was 8 trips to memory a tile, one after another (2,048 tokens, 16 heads of 128: 152 us a layer, 109 so; one tile of a decode step 11 -> 7).
         u32x4 rk[NIT], rv[NIT];
+        int id[NIT];
         const int c8 = 8 * (tid % CK), row_t = tid / CK;  // this thread's chunk of the rows row_t, row_t + 256 / CK, ...
-        auto load_tile = [&](int kb) __attribute__((always_inline)) {
+        const int ck8 = c8 < dim ? c8 : 0, cv8 = c8 < vdim ? c8 : 0;
+        auto key_of = [&](int kb, int it) __attribute__((always_inline)) {
+            const int jc = min(kb + row_t + (256 / CK) * it, k_end - 1);
+            return jc + (jc >= keep_first ? gap : 0);
+        };
+        auto page_of = [&](int j) __attribute__((always_inline)) { return page_shift >= 0 ? (j >> page_shift) : (j / page_size); };
+        auto load_ids = [&](int kb, int (&to)[NIT]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int it = 0; it < NIT; ++it) to[it] = bt[page_of(key_of(kb, it))];
+        };
+        auto load_tile = [&](int kb, const int (&page)[NIT], u32x4 (&k)[NIT], u32x4 (&v)[NIT]) __attribute__((always_inline)) {
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
-                const int jc = kb + row_t + (256 / CK) * it, j = jc + (jc >= keep_first ? gap : 0);
-                rk[it] = rv[it] = u32x4{0u, 0u, 0u, 0u};
-                if (jc < k_end) {
-                    const int pg = page_shift >= 0 ? (j >> page_shift) : (j / page_size), in_pg = j - pg * page_size;
-                    const size_t page = (size_t)bt[pg];
-                    if (c8 < dim) rk[it] = *reinterpret_cast<const u32x4 *>(kpool + ((page * G + kvh) * page_size + in_pg) * dim + c8);
-                    if (c8 < vdim) rv[it] = *reinterpret_cast<const u32x4 *>(vpool + ((page * Gv + kvh_v) * page_size + in_pg) * vdim + c8);
-                }
+                const int j = key_of(kb, it), in_pg = j - page_of(j) * page_size;
+                k[it] = *reinterpret_cast<const u32x4 *>(kpool + (((size_t)page[it] * G + kvh) * page_size + in_pg) * dim + ck8);
+                v[it] = *reinterpret_cast<const u32x4 *>(vpool + (((size_t)page[it] * Gv + kvh_v) * page_size + in_pg) * vdim + cv8);
             }
         };
-        load_tile(k_begin);
+        {
+            int first[NIT];
+            load_ids(k_begin, first);
+            load_ids(k_begin + 64, id);
+            load_tile(k_begin, first, rk, rv);
+        }
         u32x4 qb[DK8];
         const float *qrow = qbuf + ((size_t)(row_ok ? trow : r0) * H + (row_ok ? head : 0)) * dim;
 #pragma unroll
         for (int ks = 0; ks < DK8; ++ks) {
             const int d = 32 * ks + 8 * g4;
-            qb[ks] = u32x4{0u, 0u, 0u, 0u};
-            if (row_ok && d < dim) {
-                const f32x4 a = *reinterpret_cast<const f32x4 *>(qrow + d), b = *reinterpret_cast<const f32x4 *>(qrow + d + 4);
-                qb[ks] = u32x4{BF16::pack2(a[0], a[1]), BF16::pack2(a[2], a[3]), BF16::pack2(b[0], b[1]), BF16::pack2(b[2], b[3])};
-            }
+            const float *at = qrow + (d < dim ? d : 0);
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(at), b = *reinterpret_cast<const f32x4 *>(at + 4);
+            qb[ks] = u32x4{BF16::pack2(a[0], a[1]), BF16::pack2(a[2], a[3]), BF16::pack2(b[0], b[1]), BF16::pack2(b[2], b[3])};
+            if (!row_ok || d >= dim) qb[ks] = u32x4{0u, 0u, 0u, 0u};
         }
         const uint16_t *vtr = Vs + (4 * g4 + (col >> 2)) * RV + 4 * (col & 3);  // this lane's address inside a 16-key x 16-column block of values
         for (int kb = k_begin; kb < k_end; kb += 64) {
@@ -975,11 +1042,13 @@ __global__ __launch_bounds__(256) void attn_pair_tile_kernel(const float *qbuf, 
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
                 const int rw = row_t + (256 / CK) * it;
-                *reinterpret_cast<u32x4 *>(Ks + rw * RK + c8) = rk[it];
-                *reinterpret_cast<u32x4 *>(Vs + rw * RV + c8) = rv[it];
+                const bool live = kb + rw < k_end;
+                *reinterpret_cast<u32x4 *>(Ks + rw * RK + c8) = live && c8 < dim ? rk[it] : u32x4{0u, 0u, 0u, 0u};
+                *reinterpret_cast<u32x4 *>(Vs + rw * RV + c8) = live && c8 < vdim ? rv[it] : u32x4{0u, 0u, 0u, 0u};
             }
             __syncthreads();
-            if (kb + 64 < k_end) load_tile(kb + 64);
+            load_tile(kb + 64, id, rk, rv);
+            load_ids(kb + 128, id);
             // no key of the tile is masked for any row: the last one is no later than the first row, and the first one past the kept ones lies in the last row's window
             const bool inside = kb + 64 <= k_end && kb + 63 + (kb + 63 >= keep_first ? gap : 0) <= q_first &&
                                 (window <= 0 || kb + 63 < keep_first || q_last - (max(kb, keep_first) + gap) < window);
@@ -1150,46 +1219,63 @@ __global__ __launch_bounds__(256) void latent_tile_kernel(const float *qbuf, con
     const int nb = WSPLIT ? wave : 0;
     const bool row_ok = t0 + tl < len && head < H;
     const int trow = r0 + t0 + tl, qpos = pos0 + t0 + tl;
+    if (n_splits > 1 && split > 0 && k_begin >= k_end) {  // a split without keys (the sink is split 0's): the merge reads nothing but its maximum
+        if (row_ok && g4 == 0 && (!WSPLIT || wave == 0)) {
+            const size_t pi = ((size_t)trow * H + head) * n_splits + split;
+            part_ml[2 * pi] = -INFINITY;
+            part_ml[2 * pi + 1] = 0.f;
+        }
+        return;
+    }
     const bool owns_sink = sink && split == 0 && (!WSPLIT || wave == 0);
     float m_run = owns_sink ? (sinks && row_ok ? sinks[head] : 0.f) : -INFINITY, l_run = owns_sink ? 1.f : 0.f;
     f32x4 o[VT];
 #pragma unroll
     for (int v = 0; v < VT; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (k_begin < k_end) {
+        // (the next tile and the page ids of the one behind it on their way, no load behind a branch: as in attn_pair_tile_kernel; 167 -> 110 us, 13.7 -> 9.8)
         u32x4 raw[NIT];
-        auto load_tile = [&](int kb) __attribute__((always_inline)) {
+        int id[NIT];
+        auto key_of = [&](int kb, int it) __attribute__((always_inline)) { return min(kb + (tid + 256 * it) / CK, k_end - 1); };
+        auto page_of = [&](int j) __attribute__((always_inline)) { return page_shift >= 0 ? (j >> page_shift) : (j / page_size); };
+        auto load_ids = [&](int kb, int (&to)[NIT]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int it = 0; it < NIT; ++it) to[it] = bt[page_of(key_of(kb, it))];
+        };
+        auto load_tile = [&](int kb, const int (&page)[NIT], u32x4 (&to)[NIT]) __attribute__((always_inline)) {
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
-                const int q = tid + 256 * it, j = kb + q / CK, c8 = 8 * (q % CK);
-                raw[it] = u32x4{0u, 0u, 0u, 0u};
-                if (j < k_end && c8 < width) {
-                    const int pg = page_shift >= 0 ? (j >> page_shift) : (j / page_size);
-                    raw[it] = *reinterpret_cast<const u32x4 *>(pool + ((size_t)bt[pg] * page_size + (j - pg * page_size)) * width + c8);
-                }
+                const int j = key_of(kb, it), c8 = 8 * ((tid + 256 * it) % CK);
+                to[it] = *reinterpret_cast<const u32x4 *>(pool + ((size_t)page[it] * page_size + (j - page_of(j) * page_size)) * width + (c8 < width ? c8 : 0));
             }
         };
-        load_tile(k_begin);
+        {
+            int first[NIT];
+            load_ids(k_begin, first);
+            load_ids(k_begin + 64, id);
+            load_tile(k_begin, first, raw);
+        }
         u32x4 qb[DK8];
         const float *qrow = qbuf + ((size_t)(row_ok ? trow : r0) * H + (row_ok ? head : 0)) * width;
 #pragma unroll
         for (int ks = 0; ks < DK8; ++ks) {
             const int d = 32 * ks + 8 * g4;
-            qb[ks] = u32x4{0u, 0u, 0u, 0u};
-            if (row_ok && d < width) {
-                const f32x4 a = *reinterpret_cast<const f32x4 *>(qrow + d), b = *reinterpret_cast<const f32x4 *>(qrow + d + 4);
-                qb[ks] = u32x4{BF16::pack2(a[0], a[1]), BF16::pack2(a[2], a[3]), BF16::pack2(b[0], b[1]), BF16::pack2(b[2], b[3])};
-            }
+            const float *at = qrow + (d < width ? d : 0);
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(at), b = *reinterpret_cast<const f32x4 *>(at + 4);
+            qb[ks] = u32x4{BF16::pack2(a[0], a[1]), BF16::pack2(a[2], a[3]), BF16::pack2(b[0], b[1]), BF16::pack2(b[2], b[3])};
+            if (!row_ok || d >= width) qb[ks] = u32x4{0u, 0u, 0u, 0u};
         }
         const uint16_t *vtr = Ks + (4 * g4 + (col >> 2)) * RS + 4 * (col & 3);  // this lane's address inside a 16-key x 16-column block of values
         for (int kb = k_begin; kb < k_end; kb += 64) {
             __syncthreads();  // every wave is done with the previous tile
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
-                const int q = tid + 256 * it;
-                *reinterpret_cast<u32x4 *>(Ks + (q / CK) * RS + 8 * (q % CK)) = raw[it];
+                const int q = tid + 256 * it, c8 = 8 * (q % CK);
+                *reinterpret_cast<u32x4 *>(Ks + (q / CK) * RS + c8) = kb + q / CK < k_end && c8 < width ? raw[it] : u32x4{0u, 0u, 0u, 0u};
             }
             __syncthreads();
-            if (kb + 64 < k_end) load_tile(kb + 64);
+            load_tile(kb + 64, id, raw);
+            load_ids(kb + 128, id);
             const bool inside = kb + 64 <= k_end && kb + 63 <= pos0 + t0 && (window <= 0 || pos0 + min(t0 + TQ, len) - 1 - kb < window);  // no key of the tile is masked for any row
             f32x4 sc[NN];
             float m_tile = -INFINITY;
