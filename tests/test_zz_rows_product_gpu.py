@@ -1,5 +1,5 @@
-"""GPU tier: the layer-list engine's product for up to 16 rows (csrc/hybrid_kernels.h gemm_rows_kernel and its any-layout twin) against float64, at the borders of
-its forms: 4, 8 and 16 columns a block; K of a piece, a chunk, several batches of chunks and remainders; one wave to four sharing a block's K; rows behind M and
+"""GPU tier: the layer-list engine's products for up to 16 rows (csrc/hybrid_kernels.h gemm_rows_kernel and its any-layout twin) and for 17 .. 191 rows
+(gemm_mid_kernel) against float64, at the borders of their forms: 4, 8 and 16 columns a block; K of a piece, a chunk, several batches of chunks and remainders; one wave to four sharing a block's K; rows behind M and
 columns behind N.
 
 Tolerance per element: float32 sums of K products, each rounded at most twice, in any order: K * 2^-23 of sum |a w| is a bound; sqrt(K) * 2^-22 is what
@@ -43,3 +43,28 @@ def test_rows_product(dtype, M, N, K):
 def test_rows_product_any_layout(dtype, M, K, lda, offset):
     """K, row strides and alignments that 16-byte loads do not fit."""
     _product(dtype, M, 37, K, lda, offset)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "float32"])
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64, 65, 129, 191])
+@pytest.mark.parametrize("N,K", [(1, 8), (5, 72), (31, 64), (33, 256), (64, 520), (100, 2056), (1030, 136)])
+def test_mid_product(dtype, M, N, K):
+    _product(dtype, M, N, K)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [17, 40, 70])
+def test_products_that_split_their_sums_over_workgroups(n, dtype):
+    """Few columns of a long K (the feed-forward's way back): partial sums of several workgroups, in every epilogue form a layer's sums take."""
+    import layer_list_oracle as O
+    from layer_list_engine_helpers import TOL, make_engine, rel_err, tokens_for, whole
+
+    for config, make, forward in ((O.fonapel_config([O.attention_layer(ff=4096)]), O.make_fonapel_weights, O.fonapel_forward),
+                                  (O.zefapel_config([O.latent_layer(mlp=O.dense_ff(4096)), O.gla_layer(mlp=O.dense_ff(4096))]), O.make_zefapel_weights, O.zefapel_forward)):
+        W = make(config, seed=21)
+        toks = tokens_for(config, n, seed=22)
+        engine = make_engine(config, W, dtype)
+        try:
+            assert rel_err(whole(engine, toks), forward(config, W, toks)) < TOL[dtype]
+        finally:
+            engine.close()

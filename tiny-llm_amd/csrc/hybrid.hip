@@ -71,6 +71,8 @@ struct tl_hybrid {
     std::vector<float *> inv_freq;  // per mixer (2 layer + 0 / 1; those with rotary positions), device
     std::vector<float> rot_mult;    // per mixer: factor on cos and sin (rescaled frequencies)
     float *f32a = nullptr, *gates = nullptr, *idw = nullptr;  // [R, max_c] scratch (conv output, latent queries, channel decays); [R, H, 3]; [R]
+    float *mid_ws = nullptr;                                   // partial sums of products that split K over workgroups
+    size_t mid_floats = 0;
     float *chunk_ws = nullptr;                                 // chunked recurrences (recur_chunk.h): the largest layer's operands of every chunk of a step
     void *da = nullptr, *db = nullptr;                         // D-typed scratch rows: latents / low-rank inputs / attention read-out; plain queries
     hipStream_t stream = nullptr;
@@ -191,7 +193,7 @@ struct NormTail {
 
 // out (+)= A . W^T by shape: a few rows stream the weights once per column (row kernel), more go through the MFMA tile kernel
 template <typename D>
-static int linear_t(const void *A, int lda, const void *W, float *out, int ldc, int M, int N, int K, int epi, float alpha, const float *bias,
+static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, float *out, int ldc, int M, int N, int K, int epi, float alpha, const float *bias,
                     int force, hipStream_t st, int batch = 1, long sa = 0, long sw = 0, long sc = 0, NormTail *tail = nullptr, const SegSkip *skip = nullptr,
                     const BranchTail *branch = nullptr, bool *branch_done = nullptr) {
     using S = typename D::storage;
@@ -250,6 +252,31 @@ static int linear_t(const void *A, int lda, const void *W, float *out, int ldc, 
         else if (epi == 2) HY_GEMM_ROWS_C(2);
         else if (!with_tail) HY_GEMM_ROWS_C(3);
         else HY_GEMM_ROWS_C(4);
+    } else if (force == 0 && vec_ok && M < 192) {
+        // 16 to 64 rows a workgroup; K split over workgroups (at least two 128-byte pieces a wave) until every CU has two, as far as the partial sums' buffer reaches
+        const int mt = M > 48 ? 4 : (M > 32 ? 3 : 2), cols = (N + 31) / 32, mtiles = (M + 16 * mt - 1) / (16 * mt), pieces = (K + 128 / (int)sizeof(S) - 1) / (128 / (int)sizeof(S));
+        int sk = 1;
+        while (e && sk < 16 && (long)cols * mtiles * batch * sk < 2 * qmm3_num_cus() && 16 * sk <= pieces && (size_t)2 * sk * batch * M * N <= e->mid_floats) sk *= 2;
+        const dim3 grid(cols * sk, mtiles, batch), block(256), sums((unsigned)(((size_t)M * N + 255) / 256), batch);
+#define HY_MID(E, MT)                                                                                                                                          \
+    hipLaunchKernelGGL((gemm_mid_kernel<D, E, MT>), grid, block, 0, st, (const S *)A, lda, (const S *)W, out, ldc, M, N, K, alpha, bias, sk, sa, sw, sc, nw, nb, nalpha, \
+                       nout, bt, e ? e->mid_ws : (float *)nullptr)
+#define HY_MID_E(E)                                                                                                                                    \
+    do {                                                                                                                                               \
+        if (mt == 4) HY_MID(E, 4);                                                                                                                     \
+        else if (mt == 3) HY_MID(E, 3);                                                                                                                \
+        else HY_MID(E, 2);                                                                                                                             \
+        if (sk > 1)                                                                                                                                    \
+            hipLaunchKernelGGL((gemm_mid_sum_kernel<D, E>), sums, block, 0, st, e->mid_ws, sk, out, ldc, M, N, alpha, bias, sc, nw, nb, nalpha, nout, bt); \
+    } while (0)
+        if (with_branch) HY_MID_E(5);
+        else if (epi == 0) HY_MID_E(0);
+        else if (epi == 1) HY_MID_E(1);
+        else if (epi == 2) HY_MID_E(2);
+        else if (!with_tail) HY_MID_E(3);
+        else HY_MID_E(4);
+#undef HY_MID_E
+#undef HY_MID
     } else {
         dim3 grid(((M + 63) / 64) * ((N + 63) / 64), batch), block(256);
         if (with_branch) HY_GEMM(gemm_tile_kernel, 5);
@@ -755,7 +782,7 @@ static int mixer_part_t(tl_hybrid *e, size_t ri, int part, float *proj, typename
         if (L.q_rank) {
             hipLaunchKernelGGL((rms_cols_kernel<D>), dim3(rows), dim3(rows < 64 ? 512 : 128), 0, st, proj, ldp, L.q_rank, L.dq_norm_dev, c.norm_eps, (S *)e->da, L.q_rank);
             TL_CHECK_LAUNCH("hybrid latent query norm");
-            HY_TRY(linear_t<D>(e->da, L.q_rank, L.uq_dev, e->f32a, H * DQ, rows, H * DQ, L.q_rank, 0, 1.f, nullptr, 0, st));
+            HY_TRY(linear_t<D>(e, e->da, L.q_rank, L.uq_dev, e->f32a, H * DQ, rows, H * DQ, L.q_rank, 0, 1.f, nullptr, 0, st));
             q = e->f32a, ldq = H * DQ;
         }
         hipLaunchKernelGGL((latent_prep_kernel<D>), dim3(rows, H + 1), dim3(64), 0, st, q, ldq, H, L.dim, L.rot_dim, L.kv_rank, proj, ldp, kv0,
@@ -763,10 +790,10 @@ static int mixer_part_t(tl_hybrid *e, size_t ri, int part, float *proj, typename
                            inv_freq, L.rot_dims, L.rot_half, e->rot_mult[2 * layer + part], (S *)e->db, e->qbuf, (S *)run.kpool);
         TL_CHECK_LAUNCH("hybrid latent prep");
         // the keys' per-head projection moves onto the query: q_h' = W_uk,h^T q_h  -> qbuf[t, h, 0 .. kv_rank)
-        HY_TRY(linear_t<D>(e->db, H * L.dim, L.uk_t_dev, e->qbuf, H * DT, rows, L.kv_rank, L.dim, 0, 1.f, nullptr, 0, st, H, L.dim, (long)L.kv_rank * L.dim, DT));
+        HY_TRY(linear_t<D>(e, e->db, H * L.dim, L.uk_t_dev, e->qbuf, H * DT, rows, L.kv_rank, L.dim, 0, 1.f, nullptr, 0, st, H, L.dim, (long)L.kv_rank * L.dim, DT));
         HY_TRY(latent_core<D>(e, L, run.kpool, m, sh, e->da));  // one K/V head: keys [c | rotated part], values = the keys' leading kv_rank columns
         // ... and the values' onto the read-out: o_h = W_uv,h (sum_j p_j c_j)
-        HY_TRY(linear_t<D>(e->da, H * L.kv_rank, L.uv_dev, e->obuf, HV, rows, L.vdim, L.kv_rank, 0, 1.f, nullptr, 0, st, H, L.kv_rank, (long)L.vdim * L.kv_rank, L.vdim));
+        HY_TRY(linear_t<D>(e, e->da, H * L.kv_rank, L.uv_dev, e->obuf, HV, rows, L.vdim, L.kv_rank, 0, 1.f, nullptr, 0, st, H, L.kv_rank, (long)L.vdim * L.kv_rank, L.vdim));
         const size_t n = (size_t)rows * HV;
         hipLaunchKernelGGL((gate_mul_kernel<D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, e->obuf, HV, proj + g0, ldp, HV, L.gated ? 0 : 2,
                            L.gated == 2 ? L.vdim : 1, out_scale, cat, ldcat, rows);
@@ -798,7 +825,7 @@ static int mixer_part_t(tl_hybrid *e, size_t ri, int part, float *proj, typename
             const size_t na = (size_t)rows * L.a_rank, nd = (size_t)rows * H * L.dim;
             hipLaunchKernelGGL((cast_cols_kernel<D>), dim3((unsigned)((na + 255) / 256)), dim3(256), 0, st, proj, ldp, x0, L.a_rank, (S *)e->da, L.a_rank, rows);
             TL_CHECK_LAUNCH("hybrid decay input");
-            HY_TRY(linear_t<D>(e->da, L.a_rank, L.a2_dev, e->f32a, H * L.dim, rows, H * L.dim, L.a_rank, 0, 1.f, nullptr, 0, st));
+            HY_TRY(linear_t<D>(e, e->da, L.a_rank, L.a2_dev, e->f32a, H * L.dim, rows, H * L.dim, L.a_rank, 0, 1.f, nullptr, 0, st));
             hipLaunchKernelGGL(channel_decay_kernel, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, st, e->f32a, L.a2_bias_dev, H * L.dim, 1.f / L.tau, rows);
             TL_CHECK_LAUNCH("hybrid channel decay");
         } else {
@@ -898,7 +925,7 @@ static int ff_t(tl_hybrid *e, const tl_hybrid_layer &L, int rows, float *out, in
     const bool few = rows <= 8 && L.ff_kind == TL_FF_MOE && L.moe_gated && L.experts <= 64 && L.top < L.experts && L.expert_ff % 8 == 0 && L.shared_ff % 8 == 0 && e->moe_mask;
     SegSkip in_skip, out_skip;
     if (few) {
-        HY_TRY(linear_t<D>(e->h, W, (const S *)L.w_in2_dev + (size_t)2 * L.ff * W, e->proj + 2 * L.ff, nin2, rows, nin2 - 2 * L.ff, W, 0, 1.f, nullptr, 0, st));
+        HY_TRY(linear_t<D>(e, e->h, W, (const S *)L.w_in2_dev + (size_t)2 * L.ff * W, e->proj + 2 * L.ff, nin2, rows, nin2 - 2 * L.ff, W, 0, 1.f, nullptr, 0, st));
         hipLaunchKernelGGL(moe_taken_mask_kernel, dim3(1), dim3(256), 0, st, e->proj, nin2, 2 * L.ff, rows, L.experts, L.identity, L.top, L.groups, L.keep,
                            L.correction_dev, L.router_bias_dev, L.moe_router, route_opts(L), e->moe_mask);
         TL_CHECK_LAUNCH("hybrid moe taken experts");
@@ -906,14 +933,14 @@ static int ff_t(tl_hybrid *e, const tl_hybrid_layer &L, int rows, float *out, in
         in_skip.lead = out_skip.lead = L.shared_ff, in_skip.len = out_skip.len = L.expert_ff;
         in_skip.period = L.ff, in_skip.limit = 2 * L.ff, out_skip.on_k = 1;
     }
-    HY_TRY(linear_t<D>(e->h, W, L.w_in2_dev, e->proj, nin2, rows, few ? 2 * L.ff : nin2, W, 0, 1.f, nullptr, 0, st, 1, 0, 0, 0, nullptr, few ? &in_skip : nullptr));
+    HY_TRY(linear_t<D>(e, e->h, W, L.w_in2_dev, e->proj, nin2, rows, few ? 2 * L.ff : nin2, W, 0, 1.f, nullptr, 0, st, 1, 0, 0, 0, nullptr, few ? &in_skip : nullptr));
     HY_TRY(ff_act_t<D>(e, L, rows, nin2, 0, L.ff, 0));
     if (epi != 0 && L.ff_kind == TL_FF_MOE && L.identity > 0) {  // (before the experts' product: that one completes the sum and may carry the next norm, which overwrites h)
         const size_t n = (size_t)rows * W;
         hipLaunchKernelGGL((identity_axpy_kernel<D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, out, (const S *)e->h, e->idw, col, alpha, W, rows);
         TL_CHECK_LAUNCH("hybrid identity experts");
     }
-    return linear_t<D>(e->cat, L.ff, L.w_out2_dev, out, W, rows, W, L.ff, epi, alpha, col, 0, st, 1, 0, 0, 0, tail, few ? &out_skip : nullptr, branch, branch_done);
+    return linear_t<D>(e, e->cat, L.ff, L.w_out2_dev, out, W, rows, W, L.ff, epi, alpha, col, 0, st, 1, 0, 0, 0, tail, few ? &out_skip : nullptr, branch, branch_done);
 }
 
 // one run of the block with norms on both sides where the norms are Dynamic Tanh (no statistics of a row): a branch's norm, its sum, the entry of the loop pass that
@@ -950,10 +977,10 @@ static int dyt_sandwich_t(tl_hybrid *e, size_t ri, const Meta &m, const StepShap
         return TL_OK;
     };
     bool done = false;
-    HY_TRY(linear_t<D>(e->h, W, L.w_in_dev, e->proj, nmix, rows, nmix, W, L.w_in_bias_dev && !head_prep(L) ? 2 : 0, 1.f, L.w_in_bias_dev, 0, st));
+    HY_TRY(linear_t<D>(e, e->h, W, L.w_in_dev, e->proj, nmix, rows, nmix, W, L.w_in_bias_dev && !head_prep(L) ? 2 : 0, 1.f, L.w_in_bias_dev, 0, st));
     HY_TRY(mixer_t<D>(e, ri, m, sh, nmix, HV));
     const BranchTail t1 = tail(false);
-    HY_TRY(linear_t<D>(e->cat, HV, L.w_out_dev, e->y, W, rows, W, HV, 0, 1.f, nullptr, 0, st, 1, 0, 0, 0, nullptr, nullptr, &t1, &done));
+    HY_TRY(linear_t<D>(e, e->cat, HV, L.w_out_dev, e->y, W, rows, W, HV, 0, 1.f, nullptr, 0, st, 1, 0, 0, 0, nullptr, nullptr, &t1, &done));
     HY_TRY(finish(t1, done));
     if (L.ff > 0) {
         const BranchTail t2 = tail(true);
@@ -1014,7 +1041,7 @@ static int forward_t(tl_hybrid *e, const Meta &m, const StepShape &sh) {
         } else if (run.enters_pass) {  // x <- W_in [x ; x0] + step[pass]
             hipLaunchKernelGGL((pack2_kernel<D>), dim3(rows), dim3(256), 0, st, e->x, e->x0, (S *)e->cat2, W);
             TL_CHECK_LAUNCH("hybrid pack2");
-            HY_TRY(linear_t<D>(e->cat2, 2 * W, c.loop_in_dev, e->x, W, rows, W, 2 * W, 2, 1.f, c.loop_step_dev + (size_t)run.pass * W, 0, st));
+            HY_TRY(linear_t<D>(e, e->cat2, 2 * W, c.loop_in_dev, e->x, W, rows, W, 2 * W, 2, 1.f, c.loop_step_dev + (size_t)run.pass * W, 0, st));
         }
         const int nmix = layer_mixer_cols(e, run.layer), HV = layer_read_cols(e, run.layer);
         if (c.parallel_block == TL_BLOCK_POSTNORM) {
@@ -1024,9 +1051,9 @@ static int forward_t(tl_hybrid *e, const Meta &m, const StepShape &sh) {
                 hipLaunchKernelGGL((cast_rows_kernel<D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, e->x, (S *)e->h, n);
                 TL_CHECK_LAUNCH("hybrid stream cast");
             }
-            HY_TRY(linear_t<D>(e->h, W, L.w_in_dev, e->proj, nmix, rows, nmix, W, 0, 1.f, nullptr, 0, st));
+            HY_TRY(linear_t<D>(e, e->h, W, L.w_in_dev, e->proj, nmix, rows, nmix, W, 0, 1.f, nullptr, 0, st));
             HY_TRY(mixer_t<D>(e, ri, m, sh, nmix, HV));
-            HY_TRY(linear_t<D>(e->cat, HV, L.w_out_dev, e->y, W, rows, W, HV, 0, 1.f, nullptr, 0, st));
+            HY_TRY(linear_t<D>(e, e->cat, HV, L.w_out_dev, e->y, W, rows, W, HV, 0, 1.f, nullptr, 0, st));
             hipLaunchKernelGGL((postnorm_add_kernel<D>), dim3(rows), dim3(rows < 64 ? 1024 : 256), 0, st, e->x, e->y, L.norm_dev, L.norm_offset, c.norm_eps,
                                c.residual_mult, (S *)e->h, W);
             TL_CHECK_LAUNCH("hybrid norm on the mixer's output");
@@ -1058,9 +1085,9 @@ static int forward_t(tl_hybrid *e, const Meta &m, const StepShape &sh) {
             const int threads = rows < 64 ? 1024 : 256;
             // (biases: the per-head preparation of an attention layer adds them where it reads q, k and v; any other mixer gets them with the product)
             const bool prep_adds_bias = head_prep(L);
-            HY_TRY(linear_t<D>(e->h, W, L.w_in_dev, e->proj, nmix, rows, nmix, W, L.w_in_bias_dev && !prep_adds_bias ? 2 : 0, 1.f, L.w_in_bias_dev, 0, st));
+            HY_TRY(linear_t<D>(e, e->h, W, L.w_in_dev, e->proj, nmix, rows, nmix, W, L.w_in_bias_dev && !prep_adds_bias ? 2 : 0, 1.f, L.w_in_bias_dev, 0, st));
             HY_TRY(mixer_t<D>(e, ri, m, sh, nmix, HV));
-            HY_TRY(linear_t<D>(e->cat, HV, L.w_out_dev, e->y, W, rows, W, HV, 0, 1.f, nullptr, 0, st));
+            HY_TRY(linear_t<D>(e, e->cat, HV, L.w_out_dev, e->y, W, rows, W, HV, 0, 1.f, nullptr, 0, st));
             {
                 const int next = L.ff > 0 ? 2 : (side ? 1 : (Nx ? 2 : 0));
                 const float *nw = L.ff > 0 ? L.norm2_dev : (Nx ? Nx->norm_dev : nullptr);
@@ -1086,12 +1113,12 @@ static int forward_t(tl_hybrid *e, const Meta &m, const StepShape &sh) {
             }
             if (side) {  // y = W_proj (gelu_tanh(W_gate x) * e);  x += y / rms(y) * side_norm
                 const int sd = c.side_dim;
-                HY_TRY(linear_t<D>(e->h, W, L.side_gate_dev, e->proj, sd, rows, sd, W, 0, 1.f, nullptr, 0, st));
+                HY_TRY(linear_t<D>(e, e->h, W, L.side_gate_dev, e->proj, sd, rows, sd, W, 0, 1.f, nullptr, 0, st));
                 const size_t n = (size_t)rows * sd;
                 hipLaunchKernelGGL((side_act_kernel<D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, e->proj, sd, m.tokens, (const S *)c.side_embed_dev, c.side_cols,
                                    L.side_col0, sd, c.vocab, (S *)e->cat, sd, rows);
                 TL_CHECK_LAUNCH("hybrid token input");
-                HY_TRY(linear_t<D>(e->cat, sd, L.side_proj_dev, e->y, W, rows, W, sd, 0, 1.f, nullptr, 0, st));
+                HY_TRY(linear_t<D>(e, e->cat, sd, L.side_proj_dev, e->y, W, rows, W, sd, 0, 1.f, nullptr, 0, st));
                 hipLaunchKernelGGL((sandwich_add_kernel<D>), dim3(rows), dim3(threads), 0, st, e->x, e->y, L.side_norm_dev, 0.f, c.norm_eps, 1.f, (const float *)nullptr,
                                    Nx ? 2 : 0, Nx ? Nx->norm_dev : nullptr, Nx ? Nx->norm_offset : 0.f, (S *)e->h, W, (const float *)nullptr);
                 TL_CHECK_LAUNCH("hybrid norm on the token input");
@@ -1099,18 +1126,18 @@ static int forward_t(tl_hybrid *e, const Meta &m, const StepShape &sh) {
             }
         } else if (c.parallel_block == TL_BLOCK_PARALLEL) {
             const int nin = nmix + L.ff, ldcat = HV + L.ff;  // dense rows: a layer's buffers are as wide as the layer needs
-            HY_TRY(linear_t<D>(e->h, W, L.w_in_dev, e->proj, nin, rows, nin, W, 0, 1.f, nullptr, 0, st));
+            HY_TRY(linear_t<D>(e, e->h, W, L.w_in_dev, e->proj, nin, rows, nin, W, 0, 1.f, nullptr, 0, st));
             HY_TRY(mixer_t<D>(e, ri, m, sh, nin, ldcat));
             if (L.ff > 0) HY_TRY(ff_act_t<D>(e, L, rows, nin, nmix, ldcat, HV));
             // x += m * ([mixer out ; ff act] . [W_o | W_down]^T)
-            HY_TRY(linear_t<D>(e->cat, ldcat, L.w_out_dev, e->x, W, rows, W, HV + L.ff, 1, c.residual_mult, nullptr, 0, st));
+            HY_TRY(linear_t<D>(e, e->cat, ldcat, L.w_out_dev, e->x, W, rows, W, HV + L.ff, 1, c.residual_mult, nullptr, 0, st));
         } else {
             // x += m ls1 * W_o mixer(norm1 x);  x += m ls2 * ff(norm2 x)
-            HY_TRY(linear_t<D>(e->h, W, L.w_in_dev, e->proj, nmix, rows, nmix, W, 0, 1.f, nullptr, 0, st));
+            HY_TRY(linear_t<D>(e, e->h, W, L.w_in_dev, e->proj, nmix, rows, nmix, W, 0, 1.f, nullptr, 0, st));
             HY_TRY(mixer_t<D>(e, ri, m, sh, nmix, HV));
             NormTail second = (L.ff > 0 && L.norm_kind == TL_NORM_DYT) ? tail_for(L.norm2_dev, L.norm2_bias_dev, L.norm2_alpha) : NormTail{};
             NormTail *after_mixer = L.ff > 0 ? &second : &next_first;
-            HY_TRY(linear_t<D>(e->cat, HV, L.w_out_dev, e->x, W, rows, W, HV, L.ls1_dev ? 3 : 1, c.residual_mult, L.ls1_dev, 0, st, 1, 0, 0, 0, after_mixer));
+            HY_TRY(linear_t<D>(e, e->cat, HV, L.w_out_dev, e->x, W, rows, W, HV, L.ls1_dev ? 3 : 1, c.residual_mult, L.ls1_dev, 0, st, 1, 0, 0, 0, after_mixer));
             if (L.ff > 0) {
                 if (!second.done) HY_TRY(norm_t<D>(e, L.norm_kind, L.norm2_dev, L.norm2_bias_dev, L.norm2_alpha, L.norm_offset, e->h, nullptr, rows));
                 HY_TRY(ff_t<D>(e, L, rows, e->x, L.ls2_dev ? 3 : 1, c.residual_mult, L.ls2_dev, &next_first));
@@ -1129,7 +1156,7 @@ static int head_t(tl_hybrid *e, const Meta &m, int n_want, bool set_pending) {
     const tl_hybrid_config &c = e->cfg;
     if (n_want <= 0) return TL_OK;
     HY_TRY(norm_t<D>(e, c.final_norm_kind, c.final_norm_dev, c.final_norm_bias_dev, c.final_norm_alpha, c.final_norm_offset, e->hsel, m.want_rows, n_want));
-    HY_TRY(linear_t<D>(e->hsel, c.width, c.head_dev, e->logits, c.vocab, n_want, c.vocab, c.width, 0, 1.f, nullptr, 0, e->stream));
+    HY_TRY(linear_t<D>(e, e->hsel, c.width, c.head_dev, e->logits, c.vocab, n_want, c.vocab, c.width, 0, 1.f, nullptr, 0, e->stream));
     if ((c.logit_scale != 0.f && c.logit_scale != 1.f) || c.logit_softcap > 0.f) {
         const size_t n = (size_t)n_want * c.vocab;
         hipLaunchKernelGGL(logit_scale_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, e->logits, c.logit_scale != 0.f ? c.logit_scale : 1.f,
@@ -1472,6 +1499,10 @@ extern "C" int tl_hybrid_create(const tl_hybrid_config *cfg, const tl_hybrid_lay
     HY_TRY(dev_alloc(p, &e->proj, (size_t)R * e->ld_proj));
     HY_TRY(dev_alloc(p, &e->qbuf, (size_t)R * std::max(1, max_q)));
     HY_TRY(dev_alloc(p, &e->f32a, (size_t)R * std::max(1, max_c)));
+    if (R > 16) {  // (a product that splits K has at most 2 CUs' worth of 64 x 32 blocks times 2)
+        e->mid_floats = (size_t)4 * qmm3_num_cus() * 64 * 32;
+        HY_TRY(dev_alloc(p, &e->mid_ws, e->mid_floats));
+    }
     size_t chunk_floats = 0;
     for (int i = 0; i < 2 * c.num_layers; ++i) {
         const tl_hybrid_layer &L = i % 2 ? e->beside[i / 2] : e->layers[i / 2];
@@ -1811,6 +1842,6 @@ extern "C" int tl_hybrid_linear(int dtype, const void *a_dev, int lda, const voi
     TL_REQUIRE(a_dev && w_dev && out_dev, "hybrid_linear: null argument");
     TL_REQUIRE(dtype == TL_HY_BF16 || dtype == TL_HY_F32, "hybrid_linear: dtype must be bfloat16 or float32");
     TL_REQUIRE(M > 0 && N > 0 && K > 0 && lda >= K && ldc >= N, "hybrid_linear: bad shape");
-    if (dtype == TL_HY_BF16) return linear_t<BF16>(a_dev, lda, w_dev, out_dev, ldc, M, N, K, 0, 1.f, nullptr, force_kernel, (hipStream_t)stream);
-    return linear_t<F32>(a_dev, lda, w_dev, out_dev, ldc, M, N, K, 0, 1.f, nullptr, force_kernel, (hipStream_t)stream);
+    if (dtype == TL_HY_BF16) return linear_t<BF16>(nullptr, a_dev, lda, w_dev, out_dev, ldc, M, N, K, 0, 1.f, nullptr, force_kernel, (hipStream_t)stream);
+    return linear_t<F32>(nullptr, a_dev, lda, w_dev, out_dev, ldc, M, N, K, 0, 1.f, nullptr, force_kernel, (hipStream_t)stream);
 }

@@ -387,6 +387,110 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const typename D::storag
     }
 }
 
+// ---- matrix product for 17 .. 191 rows (short prompts, many decoding sequences): bound by what a CU pulls through its L1 ----
+// A wave forms 16 MT rows x 32 columns from its share of K, operands straight from memory in the matrix instruction's order (lane l: row l % 16, 16 bytes at 4 VEC
+// (l / 16) % ..): 2 + MT requests of 16 rows x 64 bytes feed 2 MT instructions, nothing is shared between waves, so nothing waits for a barrier; the next
+// 128-byte piece of every row is on its way while one is worked on.  The four waves of a workgroup take every fourth piece and meet in LDS; `sk` workgroups split K
+// further where N gives too few (2,048 columns: 64 blocks) and leave partial sums for gemm_mid_sum_kernel, added in a fixed order.
+// (64 x 64 tiles through LDS, element by element and with a branch around every load: 2,048 columns of K = 10,240, 150 rows 246 us, 47 + 5 so; whole prompts of a
+// 2048-wide Fonapel list: 20 tokens 1,333 -> 417 us, 64 1,038 -> 548, 190 1,421 -> 823; 512 wide, 20 tokens 510 -> 306.)  K % 8 == 0, 16-byte aligned rows; other layouts: gemm_tile_kernel.
+template <typename D, int EPI, int MT>
+__global__ __launch_bounds__(256) void gemm_mid_kernel(const typename D::storage *A, int lda, const typename D::storage *W, float *out, int ldc, int M, int N, int K,
+                                                       float alpha, const float *bias, int sk, long sa, long sw, long sc, const float *nw, const float *nb,
+                                                       float nalpha, typename D::storage *nout, BranchTail tail, float *partial) {
+    using S = typename D::storage;
+    constexpr int VEC = 16 / (int)sizeof(S), PIECE = 8 * VEC;  // elements of a row's 128 bytes: two requests of 4 lanes x 16 bytes
+    __shared__ f32x4 red[4][2 * MT][64];
+    A += (size_t)blockIdx.z * sa, W += (size_t)blockIdx.z * sw, out += (size_t)blockIdx.z * sc;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, lr = lane & 15;
+    const int n0 = (int)blockIdx.x / sk * 32, slice = (int)blockIdx.x % sk, m0 = (int)blockIdx.y * 16 * MT;
+    const int pieces = (K + PIECE - 1) / PIECE, per = (pieces + sk - 1) / sk, p_begin = slice * per, p_end = min(pieces, p_begin + per);
+    const S *wrow[2], *arow[MT];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) wrow[j] = W + (size_t)min(n0 + 16 * j + lr, N - 1) * K;  // (columns behind N and rows behind M are not written)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) arow[i] = A + (size_t)min(m0 + 16 * i + lr, M - 1) * lda;
+    f32x4 acc[2][MT];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Piece {
+        u32x4 w[2][2], a[MT][2];
+    };
+    auto fetch = [&](Piece &t, int p) __attribute__((always_inline)) {
+        p = min(p, pieces - 1);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = p * PIECE + u * 4 * VEC + VEC * g, at = k < K ? k : 0;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) t.w[j][u] = *reinterpret_cast<const u32x4 *>(wrow[j] + at);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) t.a[i][u] = *reinterpret_cast<const u32x4 *>(arow[i] + at);
+        }
+    };
+    auto multiply = [&](Piece &t, int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const bool in = p * PIECE + u * 4 * VEC + VEC * g < K;  // (both operands are zero behind K)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) t.w[j][u] = in ? t.w[j][u] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                t.a[i][u] = in ? t.a[i][u] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if constexpr (sizeof(S) == 2) {
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, t.w[j][u]), __builtin_bit_cast(bf16x8_t, t.a[i][u]), acc[j][i], 0, 0, 0);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(t.w[j][u][e]), __uint_as_float(t.a[i][u][e]), acc[j][i], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    };
+    Piece even, odd;
+    int p = p_begin + wave;
+    if (p < p_end) {
+        fetch(even, p);
+        for (; p < p_end; p += 8) {  // (every fetch is issued: see attn_pair_tile_kernel on branches around loads)
+            fetch(odd, p + 4);
+            multiply(even, p);
+            if (p + 4 >= p_end) break;
+            fetch(even, p + 8);
+            multiply(odd, p + 4);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) red[wave][j * MT + i][lane] = acc[j][i];
+    __syncthreads();
+    for (int b = wave; b < 2 * MT; b += 4) {  // lane: columns 4 g .. 4 g + 3 of row l % 16
+        const f32x4 v = (red[0][b][lane] + red[1][b][lane]) + (red[2][b][lane] + red[3][b][lane]);
+        const int m = m0 + 16 * (b % MT) + lr, n = n0 + 16 * (b / MT) + 4 * g;
+        if (m >= M) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (n + e >= N) continue;
+            if (sk > 1) partial[(((size_t)slice * gridDim.z + blockIdx.z) * M + m) * N + n + e] = v[e];
+            else product_out<D, EPI>(out, ldc, N, m, n + e, v[e], alpha, bias, nw, nb, nalpha, nout, tail);
+        }
+    }
+}
+template <typename D, int EPI>
+__global__ __launch_bounds__(256) void gemm_mid_sum_kernel(const float *partial, int sk, float *out, int ldc, int M, int N, float alpha, const float *bias, long sc,
+                                                           const float *nw, const float *nb, float nalpha, typename D::storage *nout, BranchTail tail) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, MN = (size_t)M * N;
+    if (i >= MN) return;
+    const float *src = partial + blockIdx.y * MN + i;
+    float v = 0.f;
+    for (int s = 0; s < sk; ++s) v += src[(size_t)s * gridDim.y * MN];
+    product_out<D, EPI>(out + (size_t)blockIdx.y * sc, ldc, N, (int)(i / N), (int)(i % N), v, alpha, bias, nw, nb, nalpha, nout, tail);
+}
+
 // the same for up to 8 rows of any K, alignment and strides: a wave per output column, element by element.  vec (float32 rows that 16-byte loads fit): 8 elements a
 // lane at a time; a matrix instruction of float32 takes 8 times a bf16 one's time, so this stays the faster form for short K and few rows (7,184 columns of
 // K = 1,024, 1 row: 7.8 us against 10.0).
