@@ -829,7 +829,7 @@ static int mixer_part_t(tl_hybrid *e, size_t ri, int part, float *proj, typename
             hipLaunchKernelGGL(channel_decay_kernel, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, st, e->f32a, L.a2_bias_dev, H * L.dim, 1.f / L.tau, rows);
             TL_CHECK_LAUNCH("hybrid channel decay");
         } else {
-            hipLaunchKernelGGL(expgate_scan_kernel, dim3(n_seqs, H), dim3(64), 0, st, proj, ldp, x0, x0 + H, L.i_bias_dev, L.f_bias_dev, L.gate_cap,
+            hipLaunchKernelGGL(expgate_scan_kernel, dim3(n_seqs, H), dim3(64 * std::min(16, (sh.max_len + 63) / 64)), 0, st, proj, ldp, x0, x0 + H, L.i_bias_dev, L.f_bias_dev, L.gate_cap,
                                m.seq_row0, m.seq_slot, run.conv_state, e->gates, H);
             TL_CHECK_LAUNCH("hybrid gate scan");
         }
@@ -842,13 +842,34 @@ static int mixer_part_t(tl_hybrid *e, size_t ri, int part, float *proj, typename
     }
     const int C = conv_channels(L);
     const size_t n = (size_t)rows * C;
-    hipLaunchKernelGGL(conv_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, proj, ldp, L.conv_dev, L.conv_taps, C, m.row_seq,
-                       m.seq_row0, m.seq_slot, run.conv_state, e->f32a, rows);
-    TL_CHECK_LAUNCH("hybrid conv");
-    if (L.conv_taps > 1) {
-        hipLaunchKernelGGL(conv_state_kernel, dim3((unsigned)(((size_t)n_seqs * C + 255) / 256)), dim3(256), 0, st, proj, ldp, L.conv_taps, C,
-                           m.seq_row0, m.seq_slot, run.conv_state, n_seqs);
-        TL_CHECK_LAUNCH("hybrid conv state");
+    // up to 8 taps by the templates (the columns in fours for a prompt); longer filters and odd columns by the general kernel
+    const bool few_taps = L.conv_taps <= 8, vec = C % 4 == 0 && ldp % 4 == 0 && (uintptr_t)proj % 16 == 0;
+    if (few_taps && sh.max_len == 1) {  // a token a sequence: the convolution and its state in one launch
+        const dim3 grid((unsigned)((n + 255) / 256));
+        if (L.conv_taps <= 4)
+            hipLaunchKernelGGL((conv_step_kernel<4>), grid, dim3(256), 0, st, proj, ldp, L.conv_dev, L.conv_taps, C, m.seq_row0, m.seq_slot, run.conv_state, e->f32a, n_seqs);
+        else
+            hipLaunchKernelGGL((conv_step_kernel<8>), grid, dim3(256), 0, st, proj, ldp, L.conv_dev, L.conv_taps, C, m.seq_row0, m.seq_slot, run.conv_state, e->f32a, n_seqs);
+        TL_CHECK_LAUNCH("hybrid conv step");
+    } else {
+        if (few_taps && vec) {
+            const dim3 grid((C / 4 + 255) / 256, (rows + 7) / 8);
+            if (L.conv_taps <= 4)
+                hipLaunchKernelGGL((conv_rows_kernel<4, 8>), grid, dim3(256), 0, st, proj, ldp, L.conv_dev, L.conv_taps, C, m.row_seq, m.seq_row0, m.seq_slot,
+                                   run.conv_state, e->f32a, rows);
+            else
+                hipLaunchKernelGGL((conv_rows_kernel<8, 8>), grid, dim3(256), 0, st, proj, ldp, L.conv_dev, L.conv_taps, C, m.row_seq, m.seq_row0, m.seq_slot,
+                                   run.conv_state, e->f32a, rows);
+        } else {
+            hipLaunchKernelGGL(conv_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, proj, ldp, L.conv_dev, L.conv_taps, C, m.row_seq, m.seq_row0,
+                               m.seq_slot, run.conv_state, e->f32a, rows);
+        }
+        TL_CHECK_LAUNCH("hybrid conv");
+        if (L.conv_taps > 1) {
+            hipLaunchKernelGGL(conv_state_kernel, dim3((unsigned)(((size_t)n_seqs * C + 255) / 256)), dim3(256), 0, st, proj, ldp, L.conv_taps, C, m.seq_row0,
+                               m.seq_slot, run.conv_state, n_seqs);
+            TL_CHECK_LAUNCH("hybrid conv state");
+        }
     }
     HY_TRY(launch_delta(e, L, run, m, n_seqs, sh.max_len, proj, ldp));
     const float *gate = proj + (size_t)C;

@@ -2375,6 +2375,77 @@ __global__ void conv_kernel(const float *proj, int ldp, const float *w, int taps
     }
     out[(size_t)t * C + c] = silu_f(acc);
 }
+// The same for up to T taps, 4 adjacent columns (C and ldp multiples of 4) and RB consecutive rows a thread: bound by memory (every input read once from
+// it, every output written once).  A thread's RB + T - 1 rows of inputs are all in flight before the first product; only rows within taps - 1 of their
+// sequence's start read the state.  Terms and order are conv_kernel's, so is every bit of the result.  2,048 rows x 6,144 columns, 4 taps:
+// 31 us (3.2 TB/s; a column and a row a thread, every row read four times: 70 us).
+template <int T, int RB>
+__global__ __launch_bounds__(256) void conv_rows_kernel(const float *proj, int ldp, const float *w, int taps, int C, const int32_t *row_seq, const int32_t *seq_row0,
+                                                        const int32_t *seq_slot, const float *state, float *out, int rows) {
+    const int c = 4 * (blockIdx.x * 256 + threadIdx.x), t0 = blockIdx.y * RB;
+    if (c >= C) return;
+    const int pad = T - taps;  // the template's taps ahead of the layer's: weight 0, input taken as 0
+    f32x4 x[RB + T - 1];
+#pragma unroll
+    for (int i = 0; i < RB + T - 1; ++i)
+        x[i] = *reinterpret_cast<const f32x4 *>(proj + (size_t)min(max(t0 - (T - 1) + i, 0), rows - 1) * ldp + c);
+    f32x4 wt[T];
+#pragma unroll
+    for (int j = 0; j < T; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = w[(size_t)(c + e) * taps + max(j - pad, 0)];
+            wt[j][e] = j < pad ? 0.f : v;
+        }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        const int t = t0 + r;
+        if (t >= rows) return;
+        const int s = row_seq[t], li = t - seq_row0[s];
+        f32x4 v[T];
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[j][e] = j < pad ? 0.f : x[r + j][e];
+        if (li < taps - 1) {
+            const float *st = state + (size_t)seq_slot[s] * (taps - 1) * C + c;
+#pragma unroll
+            for (int j = 0; j < T; ++j) {
+                const int idx = li - (T - 1) + j;
+                if (j >= pad && idx < 0) v[j] = *reinterpret_cast<const f32x4 *>(st + (size_t)(taps - 1 + idx) * C);
+            }
+        }
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < T; ++j) acc += wt[j] * v[j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = silu_f(acc[e]);
+        *reinterpret_cast<f32x4 *>(out + (size_t)t * C + c) = acc;
+    }
+}
+// Steps of one token a sequence: the thread that reads a column's inputs also moves them on, one launch instead of two.  Row t is sequence t's.
+template <int T>
+__global__ __launch_bounds__(256) void conv_step_kernel(const float *proj, int ldp, const float *w, int taps, int C, const int32_t *seq_row0,
+                                                        const int32_t *seq_slot, float *state, float *out, int n_seqs) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (size_t)n_seqs * C) return;
+    const int s = (int)(i / C), c = (int)(i % C), row = seq_row0[s], pad = T - taps;
+    float *st = state + (size_t)seq_slot[s] * (taps - 1) * C + c;
+    float v[T], wt[T];
+#pragma unroll
+    for (int j = 0; j < T - 1; ++j) v[j] = taps > 1 ? st[(size_t)min(max(j - pad, 0), max(taps - 2, 0)) * C] : 0.f;
+    v[T - 1] = proj[(size_t)row * ldp + c];
+#pragma unroll
+    for (int j = 0; j < T; ++j) wt[j] = w[(size_t)c * taps + max(j - pad, 0)];
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < T; ++j)
+        if (j >= pad) acc += wt[j] * v[j];
+    out[(size_t)row * C + c] = silu_f(acc);
+#pragma unroll
+    for (int j = 0; j < T - 1; ++j)
+        if (j >= pad) st[(size_t)(j - pad) * C] = v[j + 1];
+}
 // the convolution's inputs move on: the last taps-1 inputs after this chunk.  One thread per (sequence, channel).
 __global__ void conv_state_kernel(const float *proj, int ldp, int taps, int C, const int32_t *seq_row0, const int32_t *seq_slot, float *state,
                                   int n_seqs) {
@@ -2680,15 +2751,18 @@ __device__ __forceinline__ float logsigmoid_f(float z) { return fminf(z, 0.f) - 
 // Exponential gates with a running maximum (mLSTM).  Per (sequence, head), token by token:
 //   li = cap tanh((x_i + b_i) / cap),  lf = logsigmoid(cap tanh((x_f + b_f) / cap)),  m' = max(lf + m, li)
 //   decay a = exp(lf + m - m'),  input scale b = exp(li - m'),  floor e = exp(-m')       (m starts at 0 with the sequence)
-// m -> max(m + A, B) composes associatively ((A1, B1) then (A2, B2) = (A1 + A2, max(B1 + A2, B2))), so a wave scans 64 tokens at a time.
+// m -> max(m + A, B) composes associatively ((A1, B1) then (A2, B2) = (A1 + A2, max(B1 + A2, B2))): a wave scans 64 tokens, and the waves of a workgroup
+// (up to 16) take the running maximum across their totals one after the other, from LDS -- the sums are the ones a single wave walking the sequence forms,
+// bit for bit.  Bound by the latency of a pass: 1,900 tokens 10.5 us (one wave: 38 us).
 // proj columns i0 + h / f0 + h hold x_i / x_f.  gates: [rows, H, 3] = (a, b, e).  m_state: [slots, H].
-__global__ __launch_bounds__(64) void expgate_scan_kernel(const float *proj, int ldp, int i0, int f0, const float *i_bias, const float *f_bias, float cap,
-                                                          const int32_t *seq_row0, const int32_t *seq_slot, float *m_state, float *gates, int H) {
-    const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+__global__ __launch_bounds__(1024) void expgate_scan_kernel(const float *proj, int ldp, int i0, int f0, const float *i_bias, const float *f_bias, float cap,
+                                                            const int32_t *seq_row0, const int32_t *seq_slot, float *m_state, float *gates, int H) {
+    __shared__ float tot[2][16][2];  // two sets: a wave may write the next pass's totals while another still reads this one's
+    const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int r0 = seq_row0[s], n = seq_row0[s + 1] - r0, slot = seq_slot[s];
     float m = m_state[(size_t)slot * H + h];
-    for (int t0 = 0; t0 < n; t0 += 64) {
-        const int t = t0 + lane;
+    for (int p0 = 0, set = 0; p0 < n; p0 += blockDim.x, set ^= 1) {
+        const int t0 = p0 + 64 * wave, t = t0 + lane;
         const bool ok = t < n;
         float li = 0.f, lf = 0.f;
         if (ok) {
@@ -2704,18 +2778,24 @@ __global__ __launch_bounds__(64) void expgate_scan_kernel(const float *proj, int
                 A = pa + A;
             }
         }
-        const float m_t = fmaxf(m + A, B);
+        if (lane == 63) tot[set][wave][0] = A, tot[set][wave][1] = B;
+        __syncthreads();
+        float m_w = m;
+        for (int w = 0; w < waves; ++w) {
+            if (w == wave) m_w = m;
+            m = fmaxf(m + tot[set][w][0], tot[set][w][1]);
+        }
+        const float m_t = fmaxf(m_w + A, B);
         float m_prev = __shfl_up(m_t, 1, 64);
-        if (lane == 0) m_prev = m;
+        if (lane == 0) m_prev = m_w;
         if (ok) {
             float *g = gates + ((size_t)(r0 + t) * H + h) * 3;
             g[0] = expf(lf + m_prev - m_t);
             g[1] = expf(li - m_t);
             g[2] = expf(-m_t);
         }
-        m = __shfl(m_t, min(63, n - 1 - t0), 64);
     }
-    if (lane == 0) m_state[(size_t)slot * H + h] = m;
+    if (threadIdx.x == 0) m_state[(size_t)slot * H + h] = m;
 }
 
 // decay per key channel (gated linear attention): z[t, c] <- sigmoid(z + bias[c])^(1/tau) = exp(logsigmoid(z + bias) / tau), in place
