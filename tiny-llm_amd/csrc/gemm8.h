@@ -14,7 +14,7 @@
 //     (buffer_load ... lds, 16 bytes per lane, 8 rows per instruction, no registers): 8 instructions per lane and step; the LDS image is
 //     lane-linear, the XOR swizzle that makes the fragment reads conflict-poor is applied to the SOURCE chunk (chunk p of row r holds
 //     global chunk p ^ ((r >> 1) & 7)); rows past M / N read zeros through the buffer resource's range check;
-//   * two LDS stages (128 KB), ONE raw s_barrier per 64-wide step (a __syncthreads() would drain the DMA), the fragments of the two 32-wide
+//   * two LDS stages (128 KB; the 128-row tiles, whose steps are shorter than the way to memory, three or four), ONE raw s_barrier per 64-wide step (a __syncthreads() would drain the DMA), the fragments of the two 32-wide
 //     k-steps double-buffered in registers: a stage is refilled (tile kt + 2) as soon as every wave has read its second half, while the
 //     matrix pipe works on it;
 //   * tiles are dealt so that the workgroups of one XCD share one 256-row band of A (its L2 holds the band; the weight panels stream).
@@ -47,67 +47,94 @@ __device__ unsigned long long g8_trace[2048];
 // The tile is a parameter of the kernel body (gemm8_body.inc): WM x WN waves, TM x TN accumulator tiles (16 x 16) per wave -> BM = 16 WM TM
 // rows, BN = 16 WN TN columns.  256 x 256 = (2, 4, 8, 4);  256 x 192 = (2, 4, 8, 3) and 256 x 160 = (4, 2, 4, 5) exist because 2,048- and 4,096-row chunks against 2,560 /
 //   6,144 output columns leave a quarter to a third of the 256 CUs idle on 256 x 256 tiles (gemm8_plan picks by rounds x tile size).
-constexpr size_t gemm8_lds_bytes(int BM, int BN) { return (size_t)2 * (BM + BN) * G8_BK * 2; }
+// 128 x 160 (4, 2, 2, 5), 128 x 256 (2, 4, 4, 4) and 128 x 128 (2, 4, 4, 2): fewer rows or columns still.  Their steps take 0.5-0.8 us, less than a round trip to
+// memory under load, so with two stages every step waited for its operands: four stages (three for 128 x 256, what 160 KB hold) took 2,048 x 2,048 outputs of
+// K 10,240 on 128 x 160 tiles from 127 to 103 us, 2,000 x 2,560 of K 9,728 from 125 to 103; 128 x 128 (256 tiles instead of 208) 88 us.  On 256 x 160 a third
+// stage gave nothing where that tile is picked (174 / 176 us, 4,096 x 2,560).
+constexpr size_t gemm8_lds_bytes(int BM, int BN, int ST) { return (size_t)ST * (BM + BN) * G8_BK * 2; }
 
 #define G8_NAME gemm8_kernel_256x256
 #define G8_WM 2
 #define G8_WN 4
 #define G8_TM 8
 #define G8_TN 4
+#define G8_ST 2
 #include "gemm8_body.inc"
 #undef G8_NAME
 #undef G8_WM
 #undef G8_WN
 #undef G8_TM
 #undef G8_TN
+#undef G8_ST
 #define G8_NAME gemm8_kernel_256x192
 #define G8_WM 2
 #define G8_WN 4
 #define G8_TM 8
 #define G8_TN 3
+#define G8_ST 2
 #include "gemm8_body.inc"
 #undef G8_NAME
 #undef G8_WM
 #undef G8_WN
 #undef G8_TM
 #undef G8_TN
+#undef G8_ST
 #define G8_NAME gemm8_kernel_256x160
 #define G8_WM 4
 #define G8_WN 2
 #define G8_TM 4
 #define G8_TN 5
+#define G8_ST 2
 #include "gemm8_body.inc"
 #undef G8_NAME
 #undef G8_WM
 #undef G8_WN
 #undef G8_TM
 #undef G8_TN
+#undef G8_ST
 #define G8_NAME gemm8_kernel_128x160
 #define G8_WM 4
 #define G8_WN 2
 #define G8_TM 2
 #define G8_TN 5
+#define G8_ST 4
 #include "gemm8_body.inc"
 #undef G8_NAME
 #undef G8_WM
 #undef G8_WN
 #undef G8_TM
 #undef G8_TN
+#undef G8_ST
+#define G8_NAME gemm8_kernel_128x128
+#define G8_WM 2
+#define G8_WN 4
+#define G8_TM 4
+#define G8_TN 2
+#define G8_ST 4
+#include "gemm8_body.inc"
+#undef G8_NAME
+#undef G8_WM
+#undef G8_WN
+#undef G8_TM
+#undef G8_TN
+#undef G8_ST
 #define G8_NAME gemm8_kernel_128x256
 #define G8_WM 2
 #define G8_WN 4
 #define G8_TM 4
 #define G8_TN 4
+#define G8_ST 3
 #include "gemm8_body.inc"
 #undef G8_NAME
 #undef G8_WM
 #undef G8_WN
 #undef G8_TM
 #undef G8_TN
+#undef G8_ST
 
 // gemm8.hip
 struct Gemm8Plan {
-    int BM, BN, tiles;
+    int BM, BN, ST, tiles;
     bool ok;
 };
 Gemm8Plan gemm8_plan(int M, int N, int K);

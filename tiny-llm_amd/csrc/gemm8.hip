@@ -41,29 +41,31 @@ bool gemm8_applicable(int M, int N, int K) {
 
 int qmm3_num_cus();  // qmm3.hip
 // The tile whose grid costs the fewest (rounds over the CUs) x (outputs per tile); the narrower tiles feed their MFMAs with more LDS reads
-// per flop, priced at 3 % / 8 %.  2,048 x 6,144: 256 x 192 = 256 tiles, one round, instead of 192 on 256 x 256; 4,096 x 2,560: 256 x 160 =
-// 256 tiles instead of 160.
+// per flop, priced at 3 % to 22 %.  2,048 x 6,144: 256 x 192 = 256 tiles, one round, instead of 192 on 256 x 256; 4,096 x 2,560: 256 x 160 =
+// 256 tiles instead of 160; up to 256 tiles of 128 x 128 that one is the fastest throughout (768 x 3,072 of K 3,072: 30 us, 128 x 160 35, 256 x 160 54), of
+// 17 shapes timed on every tile the rule names the fastest each time.
 Gemm8Plan gemm8_plan(int M, int N, int K) {
     Gemm8Plan best{};
     if (!gemm8_applicable(M, N, K)) return best;
     const int cus = std::max(1, qmm3_num_cus());
 #ifndef G8_LAB_CANDS
-#define G8_LAB_CANDS 5
+#define G8_LAB_CANDS 6
 #endif
-    const struct { int bm, bn; double eff; } cand[5] = {{256, 256, 1.0}, {256, 192, 0.97}, {256, 160, 0.92}, {128, 160, 0.80}, {128, 256, 0.86}};
+    const struct { int bm, bn, st; double eff; } cand[6] = {{256, 256, 2, 1.0}, {256, 192, 2, 0.97}, {256, 160, 2, 0.92}, {128, 160, 4, 0.80}, {128, 256, 3, 0.86}, {128, 128, 4, 0.78}};
     double best_cost = 0.0;
     for (int ci = 0; ci < G8_LAB_CANDS; ++ci) {
         const auto &c = cand[ci];
+        if (K < c.st * G8_BK) continue;  // (the first stages of a tile are requested at once)
         const int tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
         const double cost = (double)((tiles + cus - 1) / cus) * c.bm * c.bn / c.eff;
-        if (!best.ok || cost < best_cost) best = Gemm8Plan{c.bm, c.bn, tiles, true}, best_cost = cost;
+        if (!best.ok || cost < best_cost) best = Gemm8Plan{c.bm, c.bn, c.st, tiles, true}, best_cost = cost;
     }
     return best;
 }
 
 template <typename KernelT>
 static int launch8(KernelT kern, const Gemm8Args &a, const Gemm8Plan &pl, hipStream_t st) {
-    const size_t lds = gemm8_lds_bytes(pl.BM, pl.BN);
+    const size_t lds = gemm8_lds_bytes(pl.BM, pl.BN, pl.ST);
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     // one workgroup per CU at most: a workgroup walks tiles b, b + grid, ... with its reduction steps running on across them (gemm8_body.inc)
     // (slots, not tiles: gemm8_body.inc deals blocks of 4 x 8 tiles to the XCDs; a ragged block's empty slots are skipped inside)
@@ -77,6 +79,7 @@ static int launch8_tile(const Gemm8Args &a, const Gemm8Plan &pl, hipStream_t st)
     if (pl.BM == 256 && pl.BN == 192) return launch8(gemm8_kernel_256x192<EPI>, a, pl, st);
     if (pl.BM == 256 && pl.BN == 160) return launch8(gemm8_kernel_256x160<EPI>, a, pl, st);
     if (pl.BM == 128 && pl.BN == 160) return launch8(gemm8_kernel_128x160<EPI>, a, pl, st);
+    if (pl.BM == 128 && pl.BN == 128) return launch8(gemm8_kernel_128x128<EPI>, a, pl, st);
     if (pl.BM == 128 && pl.BN == 256) return launch8(gemm8_kernel_128x256<EPI>, a, pl, st);
     return -1;
 }
