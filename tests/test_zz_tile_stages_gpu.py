@@ -31,3 +31,26 @@ def test_tile_stages(M, N, K):
         y = w[c:c + 16384].double()
         want, bound = a.double() @ y.T, (a.double().abs() @ y.abs().T) * (K ** 0.5 * 2.0 ** -22)
         assert bool(((out[:M, c:c + 16384].double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n", [191, 192, 700])
+def test_chunks_whose_projections_take_either_gemm(n):
+    """Chunks far below the engine's largest: every projection on the GEMM its estimate names (below 192 rows always the 4-bit one), against the float64
+    truth with the band every model-level test uses."""
+    import numpy as np
+
+    from helpers import TINY_CFG, check_against_truth, to_mlx_shaped
+    from oracle import tiny_oracle as O
+    from tiny_llm_hip.engine import DecodeEngine
+
+    weights = O.make_qwen3_weights(TINY_CFG, seed=12, sigma=0.05)
+    prompt = [int(t) for t in np.random.default_rng(n).integers(1, TINY_CFG["vocab_size"], size=n)]
+    eng = DecodeEngine(to_mlx_shaped(TINY_CFG, weights), page_size=128, num_pages=9, max_batch=1, max_prefill_rows=2048)
+    try:
+        eng.begin(0)
+        eng.prefill(0, prompt)
+        got = eng.logits(1)[0].float().cpu().numpy()
+    finally:
+        eng.close()
+    ref, truth = O.OracleQwen3(TINY_CFG, weights), O.TruthQwen3(TINY_CFG, weights)
+    check_against_truth(got[None], ref.forward(prompt)[0, -1][None], truth.forward(prompt)[0, -1][None], what=f"engine prefill of {n} rows")

@@ -73,9 +73,9 @@ struct tl_engine {
     };
     std::map<const uint32_t *, Tiled> tiled;
     size_t tiled_bytes = 0;
-    // Prefill chunks of GEMM8_MIN_ROWS (1,536) rows and more (an engine created with max_prefill_rows that large): the layer matrices once more as
+    // An engine created for chunks of GEMM8_MIN_CHUNK rows and more (max_prefill_rows): the layer matrices once more as
     // bf16 -- bf16(q * s + beta), the B operand the reference's tile GEMM forms in threadgroup memory (quantized_matmul.metal:96-249) -- for
-    // the plain bf16 GEMM of gemm8.h (256 x 256 tiles by LDS-DMA, no dequantisation in the loop).  7.3 GB at Qwen3-4B, of 288.
+    // the plain bf16 GEMM of gemm8.h (operands by LDS-DMA, no dequantisation in the loop), where gemm8_wins.  7.3 GB at Qwen3-4B, of 288.
     std::map<const uint32_t *, uint16_t *> bf16w;
     size_t bf16w_bytes = 0;
     bool use_gemm8 = true;  // tl_engine_set_option "gemm8" = 0: every chunk through the W4 GEMM (qmm.hip), the twin
@@ -363,21 +363,26 @@ static int engine_qmm(tl_engine *e, const tl_w4 &w, const uint16_t *a, uint16_t 
 // out = epilogue(a @ W^T) for any number of rows (chunked prefill, batches above 64): the reference's own op sequence --
 // W4 MFMA GEMM over the checkpoint layout (quantize.py:54-65 routes rows > 8 to the matmul path, whose tile kernel rounds
 // the dequantised weights to bf16 first), then SwiGLU / residual as separate launches.
-// From this many rows a chunk's projections run on the plain bf16 GEMM (gemm8.h).  In the lab (back-to-back launches on one weight matrix, which then sits in the
-// 256-MB Infinity Cache) gemm8 wins from ~1,500 rows; in the ENGINE every layer streams its own 202 MB of bf16 weights from HBM and the grid counts in
-// whole 256-row bands, measured at the end of round 6 (chunked prefill of 6,144 / 8,192 tokens, gemm8 / W4 GEMM, tokens/s): 1,536-row chunks 63.0k / 71.7k,
-// 2,048 83.8k / 75.6k, 3,072 77.7k / 78.0k, 4,096 100.5k / 75.9k -- so from 7 bands (until then the constant was 1,536: 12 % slower at exactly that size).
-constexpr int GEMM8_MIN_ROWS = 1792;
-static bool gemm8_wins(int M, int out_features) {
-    (void)out_features;
-    return M >= GEMM8_MIN_ROWS;
+// From this many rows of max_prefill_rows on the bf16 copies exist
+constexpr int GEMM8_MIN_CHUNK = 1792;
+// Which of a chunk's projections run on the plain bf16 GEMM (gemm8.h) where its weights exist: the estimate of its time in us, rounds over the CUs x tile x
+// reduction, against the W4 GEMM's, which is a rate and a constant (its split-K reduction takes the RMSNorm behind a residual along: 6 us that the other
+// pays as a launch).  Fitted in the engine, every layer streaming its own weights, at 256 .. 1,791 rows of two sizes; bf16 / W4 in us:
+//   6,144 x 2,560   256 rows 30 / 22, 512 29 / 31, 1,152 44 / 60, 1,791 59 / 72        19,456 x 2,560   256 38 / 47, 512 59 / 79, 1,152 111 / 145, 1,791 167 / 235
+//   2,560 x 9,728   768 89 / 60, 1,152 87 / 90, 1,280 88 / 109, 1,791 100 / 155         4,096 x 1,024    256 14 / 16, 1,024 14 / 22;  1,024 x 3,072: 1,791 32 / 26
+// (before, every projection from 1,792 rows on: 1,280 tokens of a 36-layer model 16.6 ms, now 13.5).  Fewer rows than 192 were not timed one by one.
+static bool gemm8_wins(int M, const tl_w4 &w, bool residual) {
+    if (M < 192) return false;
+    const Gemm8Plan pl = gemm8_plan(M, w.rows, w.cols);
+    if (!pl.ok) return false;
+    return 5.0 + 4.0e-7 * pl.cost * w.cols + (residual ? 6.0 : 0.0) < 12.0 + 2.8e-9 * (double)M * w.rows * w.cols;
 }
 // norm_w / norm_out / norm_done: the RMSNorm that follows an EPI_RESIDUAL projection, taken along by its split-K reduction pass where there is one
 // (small chunks on the W4 GEMM); *norm_done says whether norm_out was written -- the caller launches tl_rms_norm otherwise
 static int engine_gemm(tl_engine *e, const tl_w4 &w, const uint16_t *a, uint16_t *out, int M, int epi,
                        const uint16_t *residual, const void *norm_w = nullptr, uint16_t *norm_out = nullptr, bool *norm_done = nullptr) {
     if (norm_done) *norm_done = false;
-    if (e->use_gemm8 && gemm8_wins(M, w.rows)) {
+    if (e->use_gemm8 && gemm8_wins(M, w, epi == EPI_RESIDUAL)) {
         const auto wb = e->bf16w.find(w.weight_dev);
         if (wb != e->bf16w.end() && gemm8_applicable(M, w.rows, w.cols)) {
             Gemm8Args g{};
@@ -1488,7 +1493,7 @@ extern "C" int tl_engine_create_kv(const tl_engine_config *cfg, const tl_layer_w
         ok = ok && add_tiled(e->head());
         if (!ok) return cleanup_fail("engine_create: hipMalloc(tiled weights) failed");
     }
-    if (c.max_prefill_rows >= GEMM8_MIN_ROWS) {  // the caller asked for chunks the plain bf16 GEMM takes: expand the layer matrices once
+    if (c.max_prefill_rows >= GEMM8_MIN_CHUNK) {  // the caller asked for chunks the plain bf16 GEMM takes: expand the layer matrices once
         auto add_bf16 = [&](const tl_w4 &w) -> bool {
             if (!w.weight_dev || w.cols % 128 != 0 || e->bf16w.count(w.weight_dev) || !gemm8_applicable(c.max_prefill_rows, w.rows, w.cols)) return true;
             uint16_t *wb = nullptr;

@@ -136,6 +136,7 @@ constexpr size_t gemm8_lds_bytes(int BM, int BN, int ST) { return (size_t)ST * (
 struct Gemm8Plan {
     int BM, BN, ST, tiles;
     bool ok;
+    double cost;  // rounds over the CUs x outputs per tile / the tile's rate
 };
 Gemm8Plan gemm8_plan(int M, int N, int K);
 bool gemm8_applicable(int M, int N, int K);

@@ -58,7 +58,7 @@ Gemm8Plan gemm8_plan(int M, int N, int K) {
         if (K < c.st * G8_BK) continue;  // (the first stages of a tile are requested at once)
         const int tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
         const double cost = (double)((tiles + cus - 1) / cus) * c.bm * c.bn / c.eff;
-        if (!best.ok || cost < best_cost) best = Gemm8Plan{c.bm, c.bn, c.st, tiles, true}, best_cost = cost;
+        if (!best.ok || cost < best_cost) best = Gemm8Plan{c.bm, c.bn, c.st, tiles, true, cost}, best_cost = cost;
     }
     return best;
 }
@@ -67,10 +67,10 @@ template <typename KernelT>
 static int launch8(KernelT kern, const Gemm8Args &a, const Gemm8Plan &pl, hipStream_t st) {
     const size_t lds = gemm8_lds_bytes(pl.BM, pl.BN, pl.ST);
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    // one workgroup per CU at most: a workgroup walks tiles b, b + grid, ... with its reduction steps running on across them (gemm8_body.inc)
-    // (slots, not tiles: gemm8_body.inc deals blocks of 4 x 8 tiles to the XCDs; a ragged block's empty slots are skipped inside)
-    const int slots = (((a.M + pl.BM - 1) / pl.BM + 3) / 4 * (((a.N + pl.BN - 1) / pl.BN + 7) / 8) + 7) / 8 * 256;
-    hipLaunchKernelGGL(kern, dim3(std::min(slots, std::max(8, qmm3_num_cus() / 8 * 8))), dim3(G8_WAVES * 64), lds, st, a);
+    // one workgroup per CU at most: a workgroup walks a tile of every round with its reduction steps running on across them; whole eights, one of each per
+    // XCD (gemm8_body.inc)
+    const int grid = std::min((pl.tiles + 7) / 8 * 8, std::max(8, qmm3_num_cus() / 8 * 8));
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(G8_WAVES * 64), lds, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 template <int EPI>
