@@ -295,6 +295,9 @@ int tl_hybrid_step(tl_hybrid *e, int n_seqs, const int *slots, const int32_t *to
  * wanted row) is fed as a one-token chunk; the argmax of its logits becomes the new pending token.  `steps` steps are
  * enqueued without host involvement between them (captured in a hipGraph per batch shape where use_graph != 0). */
 int tl_hybrid_decode(tl_hybrid *e, int n_seqs, const int *slots, int steps, int use_graph);
+/* The same, up to 256 steps, with every step's ids: ids[k * n_seqs + i] = slot slots[i]'s pending token behind step k.  Pages are reserved step by step:
+ * where they run out the call fails with *done = the steps that were taken, whose ids are there.  Synchronises at the end. */
+int tl_hybrid_decode_ids(tl_hybrid *e, int n_seqs, const int *slots, int steps, int use_graph, int32_t *ids, int *done);
 int tl_hybrid_set_token(tl_hybrid *e, int slot, int32_t token);
 /* Pending token of each listed slot after synchronising. */
 int tl_hybrid_read_pending(tl_hybrid *e, int n, const int *slots, int32_t *out);

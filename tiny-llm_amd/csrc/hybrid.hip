@@ -92,6 +92,7 @@ struct tl_hybrid {
     int32_t *meta_dev = nullptr, *meta_host = nullptr;  // step metadata (host side pinned)
     int32_t *dmeta_dev = nullptr;                        // decode-loop metadata (its own copy: captured graphs point into it)
     int32_t *ctx_dev = nullptr, *pending_dev = nullptr, *argmax_dev = nullptr;
+    int32_t *hist_dev = nullptr, *hist_at_dev = nullptr;  // ids of the steps of one tl_hybrid_decode_ids call
     int32_t *last_tok_dev = nullptr;                     // [slots] the token each sequence was fed last
     tl::hy::Meta meta{}, dmeta{};
     int last_rows = 0;
@@ -1558,6 +1559,8 @@ extern "C" int tl_hybrid_create(const tl_hybrid_config *cfg, const tl_hybrid_lay
     e->dmeta = carve(e->dmeta_dev, R, c.max_slots);
     HY_TRY(dev_alloc(p, &e->table_dev, (size_t)c.max_slots * c.max_pages_per_seq));
     HY_TRY(dev_alloc(p, &e->ctx_dev, (size_t)c.max_slots, true));
+    HY_TRY(dev_alloc(p, &e->hist_dev, (size_t)DECODE_HIST * c.max_slots));
+    HY_TRY(dev_alloc(p, &e->hist_at_dev, (size_t)c.max_slots, true));
     HY_TRY(dev_alloc(p, &e->pending_dev, (size_t)c.max_slots, true));
     HY_TRY(dev_alloc(p, &e->last_tok_dev, (size_t)c.max_slots, true));
     HY_TRY(dev_alloc(p, &e->argmax_dev, (size_t)R, true));
@@ -1706,12 +1709,9 @@ extern "C" int tl_hybrid_set_token(tl_hybrid *e, int slot, int32_t token) {
     return TL_OK;
 }
 
-extern "C" int tl_hybrid_decode(tl_hybrid *e, int n_seqs, const int *slots, int steps, int use_graph) {
-    TL_REQUIRE(e && slots, "hybrid_decode: null argument");
-    TL_REQUIRE(steps >= 1, "hybrid_decode: steps must be positive");
-    HY_TRY(check_slots(e, n_seqs, slots));
+// `steps` decode steps enqueued.  goes_on: the slots, contexts and tokens on the device are those the step before left (steps of one call)
+static int decode_steps(tl_hybrid *e, int n_seqs, const int *slots, int steps, int use_graph, bool goes_on) {
     const tl_hybrid_config &c = e->cfg;
-    TL_REQUIRE(n_seqs <= c.max_rows, "hybrid_decode: more sequences than max_rows");
     std::vector<int> extra(n_seqs, steps);
     HY_TRY(reserve_all(e, n_seqs, slots, extra.data()));
     StepShape sh{n_seqs, n_seqs, 1};
@@ -1722,36 +1722,38 @@ extern "C" int tl_hybrid_decode(tl_hybrid *e, int n_seqs, const int *slots, int 
     std::vector<int> key(slot_list);  // a captured step holds its slots and its split of the key range
     key.push_back(sh.n_splits);
     key.push_back(sh.keys_per_split);
-    HY_HIP(hipStreamSynchronize(e->stream));
-    const int R = c.max_rows, S = c.max_slots;
-    if (e->dmeta_slots != slot_list) {  // static part of the decode metadata: row i <-> sequence i <-> slots[i]
-        Meta hm = carve(e->meta_host, R, S);
-        std::memset(e->meta_host, 0, meta_ints(R, S) * 4);
-        for (int i = 0; i < n_seqs; ++i) {
-            hm.row_seq[i] = i;
-            hm.seq_row0[i] = i;
-            hm.seq_slot[i] = slots[i];
-            hm.want_rows[i] = i;
-            hm.want_slot[i] = slots[i];
-        }
-        hm.seq_row0[n_seqs] = n_seqs;
-        HY_HIP(hipMemcpyAsync(e->dmeta_dev, e->meta_host, meta_ints(R, S) * 4, hipMemcpyHostToDevice, e->stream));
+    if (!goes_on) {
         HY_HIP(hipStreamSynchronize(e->stream));
-        e->dmeta_slots = slot_list;
+        const int R = c.max_rows, S = c.max_slots;
+        if (e->dmeta_slots != slot_list) {  // static part of the decode metadata: row i <-> sequence i <-> slots[i]
+            Meta hm = carve(e->meta_host, R, S);
+            std::memset(e->meta_host, 0, meta_ints(R, S) * 4);
+            for (int i = 0; i < n_seqs; ++i) {
+                hm.row_seq[i] = i;
+                hm.seq_row0[i] = i;
+                hm.seq_slot[i] = slots[i];
+                hm.want_rows[i] = i;
+                hm.want_slot[i] = slots[i];
+            }
+            hm.seq_row0[n_seqs] = n_seqs;
+            HY_HIP(hipMemcpyAsync(e->dmeta_dev, e->meta_host, meta_ints(R, S) * 4, hipMemcpyHostToDevice, e->stream));
+            HY_HIP(hipStreamSynchronize(e->stream));
+            e->dmeta_slots = slot_list;
+        }
+        std::vector<int32_t> ctx(S, 0);
+        for (int s = 0; s < S; ++s) ctx[s] = e->pool->live(s) ? e->pool->context(s) : 0;
+        HY_HIP(hipMemcpyAsync(e->ctx_dev, ctx.data(), S * 4, hipMemcpyHostToDevice, e->stream));
+        HY_HIP(hipStreamSynchronize(e->stream));
     }
-    std::vector<int32_t> ctx(S, 0);
-    for (int s = 0; s < S; ++s) ctx[s] = e->pool->live(s) ? e->pool->context(s) : 0;
-    HY_HIP(hipMemcpyAsync(e->ctx_dev, ctx.data(), S * 4, hipMemcpyHostToDevice, e->stream));
     HY_TRY(sync_table(e));
-    HY_HIP(hipStreamSynchronize(e->stream));
     auto one_step = [&]() -> int {
         hipLaunchKernelGGL(decode_meta_kernel, dim3((n_seqs + 63) / 64), dim3(64), 0, e->stream, e->dmeta.seq_slot, n_seqs, e->pending_dev, e->ctx_dev,
-                           e->dmeta.tokens, e->dmeta.row_pos, e->dmeta.seq_prev, e->last_tok_dev, 0);
+                           e->dmeta.tokens, e->dmeta.row_pos, e->dmeta.seq_prev, e->last_tok_dev, 0, e->hist_dev, e->hist_at_dev, c.max_slots);
         TL_CHECK_LAUNCH("hybrid decode meta");
         HY_TRY(forward(e, e->dmeta, sh));
         HY_TRY(head(e, e->dmeta, n_seqs, true));
         hipLaunchKernelGGL(decode_meta_kernel, dim3((n_seqs + 63) / 64), dim3(64), 0, e->stream, e->dmeta.seq_slot, n_seqs, e->pending_dev, e->ctx_dev,
-                           e->dmeta.tokens, e->dmeta.row_pos, e->dmeta.seq_prev, e->last_tok_dev, 1);
+                           e->dmeta.tokens, e->dmeta.row_pos, e->dmeta.seq_prev, e->last_tok_dev, 1, e->hist_dev, e->hist_at_dev, c.max_slots);
         TL_CHECK_LAUNCH("hybrid decode advance");
         return TL_OK;
     };
@@ -1760,6 +1762,7 @@ extern "C" int tl_hybrid_decode(tl_hybrid *e, int n_seqs, const int *slots, int 
         auto it = e->graphs.find(key);
         if (it == e->graphs.end()) {
             if (e->graphs.size() >= 32) {
+                HY_HIP(hipStreamSynchronize(e->stream));  // (a step before this one may still run one of them)
                 for (auto &g : e->graphs) (void)hipGraphExecDestroy(g.second);
                 e->graphs.clear();
             }
@@ -1791,6 +1794,38 @@ extern "C" int tl_hybrid_decode(tl_hybrid *e, int n_seqs, const int *slots, int 
     e->stats.steps += steps;
     e->stats.rows += (long)steps * n_seqs;
     return TL_OK;
+}
+
+extern "C" int tl_hybrid_decode(tl_hybrid *e, int n_seqs, const int *slots, int steps, int use_graph) {
+    TL_REQUIRE(e && slots, "hybrid_decode: null argument");
+    TL_REQUIRE(steps >= 1, "hybrid_decode: steps must be positive");
+    HY_TRY(check_slots(e, n_seqs, slots));
+    TL_REQUIRE(n_seqs <= e->cfg.max_rows, "hybrid_decode: more sequences than max_rows");
+    return decode_steps(e, n_seqs, slots, steps, use_graph, false);
+}
+
+// Step by step like as many calls of tl_hybrid_decode(.., 1, ..), without their round trips to the host (a step of a 1,024-wide Fonapel list, four slots:
+// 197 us with the ids read behind every step, 156 so): the ids stay on the device and are read once at the end.
+extern "C" int tl_hybrid_decode_ids(tl_hybrid *e, int n_seqs, const int *slots, int steps, int use_graph, int32_t *ids, int *done) {
+    TL_REQUIRE(e && slots && ids && done, "hybrid_decode_ids: null argument");
+    *done = 0;
+    TL_REQUIRE(steps >= 1 && steps <= DECODE_HIST, "hybrid_decode_ids: between 1 and 256 steps a call");
+    HY_TRY(check_slots(e, n_seqs, slots));
+    const int S = e->cfg.max_slots;
+    TL_REQUIRE(n_seqs <= e->cfg.max_rows, "hybrid_decode_ids: more sequences than max_rows");
+    hipLaunchKernelGGL(clear_ints_kernel, dim3((S + 255) / 256), dim3(256), 0, e->stream, e->hist_at_dev, S);
+    TL_CHECK_LAUNCH("hybrid decode ids");
+    int n = 0, status = TL_OK;
+    while (n < steps && (status = decode_steps(e, n_seqs, slots, 1, use_graph, n > 0)) == TL_OK) ++n;  // (a pool that runs dry ends the call behind the steps it had pages for)
+    if (n > 0) {
+        std::vector<int32_t> hist((size_t)n * S);
+        HY_HIP(hipMemcpyAsync(hist.data(), e->hist_dev, hist.size() * 4, hipMemcpyDeviceToHost, e->stream));
+        HY_HIP(hipStreamSynchronize(e->stream));
+        for (int k = 0; k < n; ++k)
+            for (int i = 0; i < n_seqs; ++i) ids[(size_t)k * n_seqs + i] = hist[(size_t)k * S + i];
+    }
+    *done = n;
+    return status;
 }
 
 extern "C" int tl_hybrid_read_pending(tl_hybrid *e, int n, const int *slots, int32_t *out) {

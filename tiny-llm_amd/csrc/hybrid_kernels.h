@@ -3231,18 +3231,30 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *logits, int v
 }
 // decode bookkeeping on the device: the step's rows are one token per listed slot; tokens come from `pending`, positions from `ctx`
 // seq_prev: the token each sequence was fed last (last_tok, by slot), which this step's token replaces
+// hist [DECODE_HIST, max_slots], hist_at [max_slots]: the ids a step left, row by row of the calls that ask for them all (a step behind the last is not kept)
+constexpr int DECODE_HIST = 256;
 __global__ void decode_meta_kernel(const int32_t *slots, int n, const int32_t *pending, int32_t *ctx, int32_t *tokens, int32_t *row_pos,
-                                   int32_t *seq_prev, int32_t *last_tok, int advance) {
+                                   int32_t *seq_prev, int32_t *last_tok, int advance, int32_t *hist, int32_t *hist_at, int max_slots) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int s = slots[i];
-    if (advance) ctx[s] += 1;
-    else {
+    if (advance) {
+        ctx[s] += 1;
+        const int at = hist_at[i];
+        if (at < DECODE_HIST) {
+            hist[(size_t)at * max_slots + i] = pending[s];
+            hist_at[i] = at + 1;
+        }
+    } else {
         tokens[i] = pending[s];
         row_pos[i] = ctx[s];
         seq_prev[i] = last_tok[s];
         last_tok[s] = pending[s];
     }
+}
+__global__ void clear_ints_kernel(int32_t *p, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0;
 }
 // the same bookkeeping of a packed step: per sequence the token fed before the step, replaced by the step's last one
 __global__ void seq_prev_kernel(const int32_t *tokens, const int32_t *seq_row0, const int32_t *seq_slot, int n, int32_t *seq_prev, int32_t *last_tok) {

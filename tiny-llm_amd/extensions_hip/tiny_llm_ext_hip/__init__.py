@@ -241,7 +241,12 @@ def _check(status: int) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream's handle, without the torch.cuda.Stream object around it (a decode step of six layers, operator by operator:
+    1.91 ms with it, 1.55 without)."""
+    return _raw_stream(torch.cuda.current_device()) if _raw_stream is not None else torch.cuda.current_stream().cuda_stream
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _require_gpu(op: str, *tensors: torch.Tensor) -> None:

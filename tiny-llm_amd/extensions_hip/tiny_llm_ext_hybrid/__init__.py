@@ -93,6 +93,7 @@ SIGNATURES = {
     "tl_hybrid_context_len": (_i, [_vp, _i]),
     "tl_hybrid_step": (_i, [_vp, _i, _P(_i), _P(ctypes.c_int32), _P(_i), _i, _P(_i)]),
     "tl_hybrid_decode": (_i, [_vp, _i, _P(_i), _i, _i]),
+    "tl_hybrid_decode_ids": (_i, [_vp, _i, _P(_i), _i, _i, _P(ctypes.c_int32), _P(_i)]),
     "tl_hybrid_set_token": (_i, [_vp, _i, ctypes.c_int32]),
     "tl_hybrid_read_pending": (_i, [_vp, _i, _P(_i), _P(ctypes.c_int32)]),
     "tl_hybrid_copy_logits": (_i, [_vp, _vp, _i]),

@@ -14,11 +14,13 @@ from __future__ import annotations
 
 import ctypes
 import os
+from array import array
 from typing import Any, Sequence
 
 import torch
 
 from ._ext import tiny_llm_ext_hip as _ext
+from .token_ids import as_int32, token_ids
 
 _lib = _ext.lib()
 
@@ -200,13 +202,13 @@ class DecodeEngine:
     def prefill(self, slot: int, tokens: Sequence[int], *, chunk: int | None = None, want_logits: bool = True) -> None:
         """Chunked prefill (reference Request.try_prefill, batch.py:48-76): all chunks append K/V, the last one
         also produces the first generated token."""
-        tokens = [int(t) for t in tokens]
+        tokens = token_ids(tokens)
         if not tokens:
             raise ValueError("prefill needs at least one token")
         chunk = self.max_prefill_rows if chunk is None else chunk  # (the largest chunk the engine was built for: 4,096-token chunks prefill at 100k tokens/s, 2,048 at 84k)
         for start in range(0, len(tokens), chunk):
             part = tokens[start:start + chunk]
-            arr = (ctypes.c_int32 * len(part))(*part)
+            arr = as_int32(part)
             last = start + chunk >= len(tokens)
             _ext.check(_lib.tl_engine_prefill(self._h, slot, arr, len(part), int(last and want_logits)))
 
@@ -216,12 +218,14 @@ class DecodeEngine:
         the slot's first generated token, like the last chunk of ``prefill``."""
         if not 1 <= len(chunks) <= 16:
             raise ValueError("prefill_packed takes between 1 and 16 chunks")
-        flat = [int(t) for _, toks, _ in chunks for t in toks]
+        flat = array("i")
+        for _, toks, _ in chunks:
+            flat.extend(token_ids(toks))
         n = len(chunks)
         slots = (ctypes.c_int * n)(*[int(c[0]) for c in chunks])
         lens = (ctypes.c_int * n)(*[len(c[1]) for c in chunks])
         want = (ctypes.c_int * n)(*[int(bool(c[2])) for c in chunks])
-        arr = (ctypes.c_int32 * len(flat))(*flat)
+        arr = as_int32(flat)
         _ext.check(_lib.tl_engine_prefill_packed(self._h, n, slots, arr, lens, want))
 
     def verify(self, slot: int, tokens: Sequence[int]) -> list[int]:

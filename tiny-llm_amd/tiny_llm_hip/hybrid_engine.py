@@ -10,14 +10,17 @@ rows -- which is what the engine's prefill and decode are made of.
 from __future__ import annotations
 
 import ctypes
+from array import array
 from typing import Any, Sequence
 
 import torch
 
 from .layer_list import LayerListConfig, pack_layer_list
+from .token_ids import as_int32, token_ids
 
 __all__ = ["HybridEngine"]
 
+_DECODE_IDS = 256  # steps a tl_hybrid_decode_ids call takes
 _FF_ACT = {"gelu_erf": 0, "gelu_tanh": 1, "silu": 2, "relu2": 3}
 _MIX = {"attention": 0, "delta": 1, "linrec": 2, "latent": 3}
 _REC = {"channel": 0, "expgate": 1, "fixed": 2}
@@ -194,7 +197,9 @@ class HybridEngine:
         n = len(entries)
         slots = (ctypes.c_int * n)(*[int(e[0]) for e in entries])
         lens = (ctypes.c_int * n)(*[len(e[1]) for e in entries])
-        flat = [int(t) for e in entries for t in e[1]]
+        flat = array("i")
+        for _, toks, _ in entries:
+            flat.extend(token_ids(toks))
         want, row0 = [], 0
         for _, toks, places in entries:
             for p in places:
@@ -202,7 +207,7 @@ class HybridEngine:
                     raise ValueError("step: a wanted place lies outside its chunk")
                 want.append(row0 + int(p))
             row0 += len(toks)
-        tokens = (ctypes.c_int32 * max(1, len(flat)))(*flat)
+        tokens = as_int32(flat)
         want_c = (ctypes.c_int * max(1, len(want)))(*want)
         self._ext.check(self._lib.tl_hybrid_step(self._h, n, slots, tokens, lens, len(want), want_c))
         self._rows = len(want)
@@ -210,7 +215,7 @@ class HybridEngine:
 
     def prefill(self, slot: int, tokens: Sequence[int], *, chunk: int | None = None, want_logits: bool = True) -> None:
         """Chunked prefill of one slot; the last chunk leaves the last row's logits and the first generated token."""
-        tokens = [int(t) for t in tokens]
+        tokens = token_ids(tokens)
         if not tokens:
             raise ValueError("prefill needs at least one token")
         chunk = min(self.max_prefill_rows, chunk or self.max_prefill_rows)
@@ -234,10 +239,13 @@ class HybridEngine:
         if not slots:
             return
         arr = (ctypes.c_int * len(slots))(*slots)
-        for _ in range(steps):  # one captured step per call: the ids of every step are kept for read_tokens
-            self._ext.check(self._lib.tl_hybrid_decode(self._h, len(slots), arr, 1, int(use_graph)))
-            for s, tok in zip(slots, self.read_pending_slots(slots)):
-                self._produced.setdefault(s, []).append(tok)
+        ids, done, left = (ctypes.c_int32 * (len(slots) * _DECODE_IDS))(), ctypes.c_int(0), len(range(steps))
+        while left:
+            status = self._lib.tl_hybrid_decode_ids(self._h, len(slots), arr, min(left, _DECODE_IDS), int(use_graph), ids, ctypes.byref(done))
+            for i, s in enumerate(slots):
+                self._produced.setdefault(s, []).extend(ids[i:done.value * len(slots):len(slots)])
+            self._ext.check(status)
+            left -= done.value
         self._rows = len(slots)
 
     def decode_free_running(self, steps: int, slots: Sequence[int], use_graph: bool = True) -> None:
