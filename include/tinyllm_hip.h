@@ -91,6 +91,12 @@ int tl_rms_norm(const void *x, const void *weight, void *out, int rows, int dim,
 int tl_rope(const void *x, const int32_t *offsets, void *out, int B, int L, int H, int D, int dims, float base,
             int traditional, tl_dtype dtype, void *stream);
 
+/* ---- the q and k of an attention layer: tl_rms_norm over each head's 128 dims, then tl_rope over all of them (half-split pairs), bit for bit ----
+ * q [B,L,Hq,128], k [B,L,Hk,128] -> q_out [B,Hq,L,128], k_out [B,Hk,L,128]; offsets [B] int32 on the device, or NULL: `offset` for
+ * every batch row.  bfloat16, everything on 16 bytes. */
+int tl_qk_norm_rope(const void *q, const void *k, const void *q_weight, const void *k_weight, const int32_t *offsets, int offset, void *q_out,
+                    void *k_out, int B, int L, int q_heads, int k_heads, int D, float q_eps, float k_eps, float base, tl_dtype dtype, void *stream);
+
 /* ---- replaces swiglu (week2_kernels.cpp:57-63,158-174) ---------------------- */
 int tl_swiglu(const void *gate, const void *up, void *out, size_t size, tl_dtype dtype, void *stream);
 
@@ -113,6 +119,10 @@ int tl_gather_quantized_matvec(const void *scales, const void *biases, const voi
  * pages [P,H,page_size,D] (written IN PLACE), values [1,H,length,D]. */
 int tl_paged_cache_update(void *pages, const void *values, int num_pages, int heads, int page_size, int head_dim,
                           int length, int page_id, int start, tl_dtype dtype, void *stream);
+
+/* Both of a layer's page arrays at once, from [1,H,length,D] views with contiguous rows: head and token strides in BYTES, everything on 16 bytes. */
+int tl_paged_cache_write(void *key_pages, void *value_pages, const void *key, const void *value, long k_head, long k_token, long v_head, long v_token,
+                         int num_pages, int heads, int page_size, int head_dim, int length, int page_id, int start, tl_dtype dtype, void *stream);
 
 /* ---- replaces paged_attention (paged_attention.cpp:77-225) ------------------
  * q,out [N=B*Hq, L, D]; key_pages,value_pages [P,Hkv,page_size,D];

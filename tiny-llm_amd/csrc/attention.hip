@@ -131,6 +131,19 @@ __global__ __launch_bounds__(256) void paged_cache_update_kernel(const char *__r
         *reinterpret_cast<uint16_t *>(pages + dst) = *reinterpret_cast<const uint16_t *>(values + src);
     }
 }
+// K and V of one page's slots in one launch (blockIdx.y), straight from [H, length, D] views whose rows are contiguous: head and token strides in bytes, 16 bytes
+// a thread.  Four launches before (two copies to contiguous memory, two scatters): 1,000 tokens of 8 heads over 8 pages 32 launches a layer, now 8.
+__global__ __launch_bounds__(256) void paged_cache_write_kernel(const char *__restrict__ key, const char *__restrict__ value, long k_head, long k_token, long v_head,
+                                                                long v_token, char *__restrict__ key_pages, char *__restrict__ value_pages, int heads, int length,
+                                                                int vecs, int page_size, int page_id, int start) {
+    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= (long)heads * length * vecs) return;
+    const int within = (int)(idx % vecs), token = (int)(idx / vecs % length), head = (int)(idx / vecs / length);
+    const bool v = blockIdx.y != 0;
+    const long dst = ((((long)page_id * heads + head) * page_size + start + token) * vecs + within) * 16;
+    const long src = (v ? head * v_head + token * v_token : head * k_head + token * k_token) + within * 16;
+    *reinterpret_cast<uint4 *>((v ? value_pages : key_pages) + dst) = *reinterpret_cast<const uint4 *>((v ? value : key) + src);
+}
 
 // ---------------------------------------------------------------------------
 // FP8 (E4M3) pages (kv8.h; no reference counterpart): the quantising twin of the scatter above -- rows of 128 bf16 values
@@ -958,6 +971,23 @@ extern "C" int tl_paged_cache_update(void *pages, const void *values, int num_pa
                            (const char *)values, (char *)pages, heads, length, row_bytes, page_size, page_id, start);
     }
     TL_CHECK_LAUNCH("paged_cache_update");
+    return TL_OK;
+}
+
+extern "C" int tl_paged_cache_write(void *key_pages, void *value_pages, const void *key, const void *value, long k_head, long k_token, long v_head, long v_token,
+                                    int num_pages, int heads, int page_size, int head_dim, int length, int page_id, int start, tl_dtype dtype, void *stream) {
+    TL_REQUIRE(dtype == TL_F32 || dtype == TL_BF16, "paged_cache_write: pages and values must have the same float32 or bfloat16 dtype");
+    TL_REQUIRE(key_pages && value_pages && key && value, "paged_cache_write: null pointer");
+    TL_REQUIRE(heads > 0 && page_size > 0 && head_dim > 0 && length >= 0, "paged_cache_write: expected pages [P, H, page_size, D] and values [1, H, length, D]");
+    TL_REQUIRE(page_id >= 0 && page_id < num_pages && start >= 0 && start + length <= page_size, "paged_cache_write: destination slice is outside page storage");
+    const long row_bytes = (long)head_dim * (dtype == TL_F32 ? 4 : 2);
+    TL_REQUIRE((row_bytes | k_head | k_token | v_head | v_token) % 16 == 0 && ((uintptr_t)key_pages | (uintptr_t)value_pages | (uintptr_t)key | (uintptr_t)value) % 16 == 0,
+               "paged_cache_write: rows start on 16 bytes");
+    if (length == 0) return TL_OK;
+    const int vecs = (int)(row_bytes / 16);
+    hipLaunchKernelGGL(paged_cache_write_kernel, dim3(ceil_div((long)heads * length * vecs, 256), 2), dim3(256), 0, (hipStream_t)stream, (const char *)key,
+                       (const char *)value, k_head, k_token, v_head, v_token, (char *)key_pages, (char *)value_pages, heads, length, vecs, page_size, page_id, start);
+    TL_CHECK_LAUNCH("paged_cache_write");
     return TL_OK;
 }
 

@@ -69,6 +69,8 @@ _SIGNATURES = {
     "tl_rope": (_c_int, [_c_void_p] * 3 + [_c_int] * 5 + [_c_float, _c_int, _c_int, _c_void_p]),
     "tl_swiglu": (_c_int, [_c_void_p] * 3 + [_c_size_t, _c_int, _c_void_p]),
     "tl_decode_attention": (_c_int, [_c_void_p] * 5 + [_c_int] * 6 + [_c_float, _c_int, _c_int, _c_int, _c_void_p]),
+    "tl_qk_norm_rope": (_c_int, [_c_void_p] * 5 + [_c_int] + [_c_void_p] * 2 + [_c_int] * 5 + [_c_float] * 3 + [_c_int, _c_void_p]),
+    "tl_paged_cache_write": (_c_int, [_c_void_p] * 4 + [ctypes.c_long] * 4 + [_c_int] * 8 + [_c_void_p]),
     "tl_paged_cache_update": (_c_int, [_c_void_p] * 2 + [_c_int] * 8 + [_c_void_p]),
     "tl_paged_attention": (
         _c_int,
@@ -447,6 +449,27 @@ def rope(
     return out
 
 
+def qk_norm_rope_takes(q: torch.Tensor, k: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.Tensor) -> bool:
+    """Whether ``qk_norm_rope`` has a kernel for these: contiguous bfloat16 [B, L, H, 128] rows on 16 bytes, weights like them, one device."""
+    ts = (q, k, q_weight, k_weight)
+    return (q.dtype is torch.bfloat16 and q.dim() == 4 and k.dim() == 4 and q.shape[:2] == k.shape[:2] and q.shape[3] == k.shape[3] == 128
+            and q.numel() > 0 and k.numel() > 0 and tuple(q_weight.shape) == tuple(k_weight.shape) == (128,)
+            and all(t.is_cuda and t.dtype == q.dtype and t.device == q.device and t.is_contiguous() and _ptr(t) % 16 == 0 for t in ts))
+
+
+def qk_norm_rope(q, k, q_weight, k_weight, offset, q_eps: float, k_eps: float, base: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """rms_norm over each head, then rope over all 128 dims, of a layer's q [B,L,Hq,128] and k [B,L,Hk,128], as [B,H,L,128]: the two operators' results
+    bit for bit in one launch (tl_qk_norm_rope).  ``offset``: an int, or one int32 per batch row on the device.  Callers ask qk_norm_rope_takes first."""
+    B, L, Hq, D = q.shape
+    Hk = k.shape[2]
+    q_out = torch.empty((B, Hq, L, D), dtype=q.dtype, device=q.device)
+    k_out = torch.empty((B, Hk, L, D), dtype=k.dtype, device=k.device)
+    per_row = isinstance(offset, torch.Tensor)
+    _check(_lib.tl_qk_norm_rope(_ptr(q), _ptr(k), _ptr(q_weight), _ptr(k_weight), _ptr(offset) if per_row else None, 0 if per_row else offset, _ptr(q_out),
+                                _ptr(k_out), B, L, Hq, Hk, D, float(q_eps), float(k_eps), float(base), _DTYPES[q.dtype], _stream()))
+    return q_out, k_out
+
+
 def swiglu(gate: torch.Tensor, up: torch.Tensor, stream=None) -> torch.Tensor:
     """``silu(gate) * up`` (reference week2_kernels.cpp:57-63)."""
     _require_float(gate, "swiglu")
@@ -524,6 +547,25 @@ def paged_cache_update(pages: torch.Tensor, values: torch.Tensor, page_id: int, 
                                    int(start), _DTYPES[pages.dtype], _stream())
     )
     return pages
+
+
+def paged_cache_write(key_pages: torch.Tensor, value_pages: torch.Tensor, key: torch.Tensor, value: torch.Tensor, page_id: int, start: int) -> bool:
+    """``key`` / ``value`` [1,H,len,D], any head and token strides, into both page arrays in one launch (tl_paged_cache_write).  False, and nothing written,
+    for what that kernel does not take: the caller goes through ``paged_cache_update`` then, whose checks and errors hold for both."""
+    ts = (key_pages, value_pages, key, value)
+    P, H, page_size, D = key_pages.shape
+    size = key.element_size()
+    if (value_pages.shape != key_pages.shape or key.shape != value.shape or key.dim() != 4 or key.shape[0] != 1 or key.shape[1] != H or key.shape[3] != D
+            or not 0 <= page_id < P or start < 0 or start + key.shape[2] > page_size or key.dtype not in (torch.float32, torch.bfloat16)
+            or D * size % 16 or not all(t.is_cuda and t.dtype == key.dtype and t.device == key.device and _ptr(t) % 16 == 0 for t in ts)
+            or not key_pages.is_contiguous() or not value_pages.is_contiguous()):
+        return False
+    (_, kh, kt, kd), (_, vh, vt, vd) = key.stride(), value.stride()
+    if kd != 1 or vd != 1 or any(s * size % 16 for s in (kh, kt, vh, vt)):
+        return False
+    _check(_lib.tl_paged_cache_write(_ptr(key_pages), _ptr(value_pages), _ptr(key), _ptr(value), kh * size, kt * size, vh * size, vt * size, P, H, page_size, D,
+                                     key.shape[2], int(page_id), int(start), _DTYPES[key.dtype], _stream()))
+    return True
 
 
 def paged_attention(

@@ -189,8 +189,8 @@ class TinyKvPagedPool:
         self.copied_bytes_on_growth = 0
 
     def write_page_slice(self, page_id: int, start: int, key: torch.Tensor, value: torch.Tensor) -> None:
-        """Write ``key``/``value`` [1, H, len, D] into slots [start, start+len) of one page (two scatter launches,
-        reference paged_kv_cache.py:196-234)."""
+        """Write ``key``/``value`` [1, H, len, D] into slots [start, start+len) of one page (one launch where the extension takes
+        the views as they are, two scatters of contiguous copies otherwise; reference paged_kv_cache.py:196-234)."""
         self.validate_page_chunk(key, value)
         if key.shape[2] > self.page_size:
             raise ValueError("Paged K/V writes cannot exceed one physical page")
@@ -201,6 +201,8 @@ class TinyKvPagedPool:
         if start < 0 or start + key.shape[2] > self.page_size:
             raise ValueError("Paged K/V write is outside page storage")
         self._ensure_page_storage(key, value)
+        if key.is_cuda and tiny_llm_ext_hip.paged_cache_write(self._key_pages, self._value_pages, key, value, page_id, start):
+            return
         self._key_pages = tiny_llm_ext_hip.paged_cache_update(self._key_pages, key.contiguous(), page_id, start)
         self._value_pages = tiny_llm_ext_hip.paged_cache_update(self._value_pages, value.contiguous(), page_id, start)
 

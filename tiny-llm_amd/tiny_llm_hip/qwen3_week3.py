@@ -10,7 +10,7 @@ from .kv_cache import TinyKvCache
 from .moe import Moe
 from .paged_kv_cache import TinyKvPagedCache, TinyKvPagedPool
 from .quantize import QuantizedWeights, quantized_linear
-from .week2_kernels import FastRMSNorm, FastRoPE, decode_attention_custom, scaled_dot_product_attention, swiglu
+from .week2_kernels import FastRMSNorm, FastRoPE, decode_attention_custom, norm_and_rotate, scaled_dot_product_attention, swiglu
 
 
 class Qwen3MultiHeadAttention:
@@ -32,12 +32,10 @@ class Qwen3MultiHeadAttention:
 
     def __call__(self, x, offsets, cache: TinyKvCache, mask=None) -> torch.Tensor:
         B, L, _ = x.shape
-        q = self.q_norm(quantized_linear(x, self.wq).reshape(B, L, self.num_heads, self.head_dim))
-        k = self.k_norm(quantized_linear(x, self.wk).reshape(B, L, self.num_kv_heads, self.head_dim))
-        v = quantized_linear(x, self.wv).reshape(B, L, self.num_kv_heads, self.head_dim)
-        q = self.rope(q, offset=offsets).transpose(1, 2)
-        k = self.rope(k, offset=offsets).transpose(1, 2)
-        v = v.transpose(1, 2)
+        q = quantized_linear(x, self.wq).reshape(B, L, self.num_heads, self.head_dim)
+        k = quantized_linear(x, self.wk).reshape(B, L, self.num_kv_heads, self.head_dim)
+        v = quantized_linear(x, self.wv).reshape(B, L, self.num_kv_heads, self.head_dim).transpose(1, 2)
+        q, k = norm_and_rotate(q, k, self.q_norm, self.k_norm, self.rope, offsets)
         if self.use_paged_attention:
             meta = cache.update_and_fetch_paged(k, v, mask_length=L, mask=mask)
             mixed = paged_attention(

@@ -37,7 +37,8 @@ class FastRoPE:
         self.base = base
         self.traditional = traditional
 
-    def __call__(self, x: torch.Tensor, offset: int | list[int] | torch.Tensor = 0) -> torch.Tensor:
+    def _offsets(self, x: torch.Tensor, offset: int | list[int] | torch.Tensor) -> torch.Tensor:
+        """One int32 offset per batch row, on x's device."""
         batch = x.shape[0]
         if isinstance(offset, int):
             offsets = torch.full((batch,), offset, dtype=torch.int32, device=x.device)
@@ -51,7 +52,22 @@ class FastRoPE:
             raise ValueError("FastRoPE needs one offset per batch row")
         else:
             offsets = offset.to(device=x.device, dtype=torch.int32)
-        return tiny_llm_ext_hip.rope(x.contiguous(), offsets.contiguous(), self.dims, self.base, self.traditional)
+        return offsets.contiguous()
+
+    def __call__(self, x: torch.Tensor, offset: int | list[int] | torch.Tensor = 0) -> torch.Tensor:
+        return tiny_llm_ext_hip.rope(x.contiguous(), self._offsets(x, offset), self.dims, self.base, self.traditional)
+
+
+def norm_and_rotate(q: torch.Tensor, k: torch.Tensor, q_norm, k_norm, rope, offset) -> tuple[torch.Tensor, torch.Tensor]:
+    """``rope(norm(x), offset=offset).transpose(1, 2)`` of a layer's q and k [B, L, H, D].  One launch instead of six, same bits, where both norms are
+    FastRMSNorm over 128 dims, the rotation FastRoPE over all of them in half-split pairs, and the rows as the kernel takes them; operator by operator else."""
+    if q.is_cuda and type(q_norm) is type(k_norm) is FastRMSNorm and type(rope) is FastRoPE and rope.dims == 128 and not rope.traditional:
+        wq, wk = q_norm.weight.to(q.dtype).contiguous(), k_norm.weight.to(k.dtype).contiguous()
+        if tiny_llm_ext_hip.qk_norm_rope_takes(q, k, wq, wk):
+            if not (isinstance(offset, int) and -2 ** 31 <= offset < 2 ** 31):
+                offset = rope._offsets(q, offset)
+            return tiny_llm_ext_hip.qk_norm_rope(q, k, wq, wk, offset, q_norm.eps, k_norm.eps, rope.base)
+    return rope(q_norm(q), offset=offset).transpose(1, 2), rope(k_norm(k), offset=offset).transpose(1, 2)
 
 
 def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
