@@ -196,7 +196,7 @@ struct NormTail {
 template <typename D>
 static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, float *out, int ldc, int M, int N, int K, int epi, float alpha, const float *bias,
                     int force, hipStream_t st, int batch = 1, long sa = 0, long sw = 0, long sc = 0, NormTail *tail = nullptr, const SegSkip *skip = nullptr,
-                    const BranchTail *branch = nullptr, bool *branch_done = nullptr) {
+                    const BranchTail *branch = nullptr, bool *branch_done = nullptr, const BranchTail *act = nullptr, bool *act_done = nullptr) {
     using S = typename D::storage;
     if (M <= 0 || N <= 0 || batch <= 0) return TL_OK;
     const int vec_ok = (K % 8 == 0) && (lda % 8 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0) && sa % 8 == 0 && sw % 8 == 0;
@@ -210,7 +210,12 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
             Gemm8Args g{};
             g.a = (const uint16_t *)A, g.w = (const uint16_t *)W, g.M = M, g.N = N, g.K = K, g.out_f32 = out, g.alpha = alpha;
             if (epi == 3) g.col_scale = bias;
-            if (launch_gemm8_bf16(g, (epi == 1 || epi == 3) ? EPI_F32_AXPY : EPI_F32_STORE, st) == 0) {
+            const bool act8 = act && epi == 0 && act->act_from % 4 == 0 && act->act_ld % 4 == 0 && ((uintptr_t)act->bias % 16 | (uintptr_t)act->h % 8) == 0;
+            if (act8) {
+                g.act_out = (uint16_t *)act->h, g.act_bias = act->bias, g.act_from = act->act_from, g.act_ld = act->act_ld, g.act_kind = act->act_kind;
+                *act_done = true;
+            }
+            if (launch_gemm8_bf16(g, act8 ? EPI_F32_ACT : ((epi == 1 || epi == 3) ? EPI_F32_AXPY : EPI_F32_STORE), st) == 0) {
                 if (epi == 2) {
                     const size_t n = (size_t)M * N;
                     hipLaunchKernelGGL(add_rowvec_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, out, bias, N, M);
@@ -219,6 +224,7 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
                 return TL_OK;
             }
         }
+        if (act_done) *act_done = false;
         TL_REQUIRE(force != 3, "hybrid linear: the 256-wide tile GEMM does not take this shape");
     }
     const bool with_tail = tail && tail->out && epi == 3 && batch == 1 && ldc == N;
@@ -226,7 +232,8 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
     const float nalpha = with_tail ? tail->alpha : 0.f;
     S *nout = with_tail ? (S *)tail->out : nullptr;
     const bool with_branch = branch && epi == 0 && batch == 1 && ldc == N;  // (the product forms a whole branch: its tail leaves with it, `out` is not written)
-    const BranchTail bt = with_branch ? *branch : BranchTail{};
+    const bool with_act = act && epi == 0 && batch == 1 && ldc == N && !skip && !with_branch;
+    const BranchTail bt = with_branch ? *branch : (with_act ? *act : BranchTail{});
 #define HY_GEMM(KERN, E) \
     hipLaunchKernelGGL((KERN<D, E>), grid, block, 0, st, (const S *)A, lda, (const S *)W, out, ldc, M, N, K, alpha, bias, vec_ok, sa, sw, sc, nw, nb, nalpha, nout, bt)
 #define HY_GEMM_ROWS(KERN, E) \
@@ -248,6 +255,7 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
         dim3 grid(blocked ? (blocks * ks + 3) / 4 : (N + 3) / 4, batch), block(256);
         const SegSkip sk = skip ? *skip : SegSkip{};
         if (with_branch) HY_GEMM_ROWS_C(5);
+        else if (with_act) HY_GEMM_ROWS_C(6);
         else if (epi == 0) HY_GEMM_ROWS_C(0);
         else if (epi == 1) HY_GEMM_ROWS_C(1);
         else if (epi == 2) HY_GEMM_ROWS_C(2);
@@ -271,6 +279,7 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
             hipLaunchKernelGGL((gemm_mid_sum_kernel<D, E>), sums, block, 0, st, e->mid_ws, sk, out, ldc, M, N, alpha, bias, sc, nw, nb, nalpha, nout, bt); \
     } while (0)
         if (with_branch) HY_MID_E(5);
+        else if (with_act) HY_MID_E(6);
         else if (epi == 0) HY_MID_E(0);
         else if (epi == 1) HY_MID_E(1);
         else if (epi == 2) HY_MID_E(2);
@@ -281,6 +290,7 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
     } else {
         dim3 grid(((M + 63) / 64) * ((N + 63) / 64), batch), block(256);
         if (with_branch) HY_GEMM(gemm_tile_kernel, 5);
+        else if (with_act) HY_GEMM(gemm_tile_kernel, 6);
         else if (epi == 0) HY_GEMM(gemm_tile_kernel, 0);
         else if (epi == 1) HY_GEMM(gemm_tile_kernel, 1);
         else if (epi == 2) HY_GEMM(gemm_tile_kernel, 2);
@@ -292,6 +302,7 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
 #undef HY_GEMM_ROWS_C
     if (with_tail) tail->done = true;
     if (branch_done) *branch_done = with_branch;
+    if (act_done) *act_done = with_act;
     TL_CHECK_LAUNCH("hybrid linear");
     return TL_OK;
 }
@@ -935,6 +946,16 @@ static int ff_act_t(tl_hybrid *e, const tl_hybrid_layer &L, int rows, int ldp, i
     return TL_OK;
 }
 
+// The activation of a feed-forward without gates or experts leaves with the product that forms its columns (from `up0` on), into cat: one launch and a float32
+// round trip of those columns less (2,048 rows x 8,192: 17 us of their own; a step of four rows 3 us).  h NULL: ff_act_t behind the product.
+template <typename D>
+static BranchTail plain_act(const tl_hybrid *e, const tl_hybrid_layer &L, int up0, int ldcat, int col0) {
+    BranchTail t;
+    if (L.ff <= 0 || L.ff_kind == TL_FF_MOE || L.ff_kind == TL_FF_GATED) return t;
+    t.h = (typename D::storage *)e->cat + col0, t.bias = L.ff_in_bias_dev, t.act_from = up0, t.act_ld = ldcat, t.act_kind = L.ff_act;
+    return t;
+}
+
 // a feed-forward of its own matrices on the D rows e->h: out (+)= (epi, alpha, col as in linear_t) its result.  Where the result is added (epi 1 / 3) the
 // identity experts' part is added too; a caller that takes the bare result (epi 0) adds it itself.
 template <typename D>
@@ -955,8 +976,11 @@ static int ff_t(tl_hybrid *e, const tl_hybrid_layer &L, int rows, float *out, in
         in_skip.lead = out_skip.lead = L.shared_ff, in_skip.len = out_skip.len = L.expert_ff;
         in_skip.period = L.ff, in_skip.limit = 2 * L.ff, out_skip.on_k = 1;
     }
-    HY_TRY(linear_t<D>(e, e->h, W, L.w_in2_dev, e->proj, nin2, rows, few ? 2 * L.ff : nin2, W, 0, 1.f, nullptr, 0, st, 1, 0, 0, 0, nullptr, few ? &in_skip : nullptr));
-    HY_TRY(ff_act_t<D>(e, L, rows, nin2, 0, L.ff, 0));
+    bool act_done = false;
+    const BranchTail act = plain_act<D>(e, L, 0, L.ff, 0);
+    HY_TRY(linear_t<D>(e, e->h, W, L.w_in2_dev, e->proj, nin2, rows, few ? 2 * L.ff : nin2, W, 0, 1.f, nullptr, 0, st, 1, 0, 0, 0, nullptr, few ? &in_skip : nullptr,
+                       nullptr, nullptr, act.h ? &act : nullptr, &act_done));
+    if (!act_done) HY_TRY(ff_act_t<D>(e, L, rows, nin2, 0, L.ff, 0));
     if (epi != 0 && L.ff_kind == TL_FF_MOE && L.identity > 0) {  // (before the experts' product: that one completes the sum and may carry the next norm, which overwrites h)
         const size_t n = (size_t)rows * W;
         hipLaunchKernelGGL((identity_axpy_kernel<D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, out, (const S *)e->h, e->idw, col, alpha, W, rows);
@@ -1148,9 +1172,12 @@ static int forward_t(tl_hybrid *e, const Meta &m, const StepShape &sh) {
             }
         } else if (c.parallel_block == TL_BLOCK_PARALLEL) {
             const int nin = nmix + L.ff, ldcat = HV + L.ff;  // dense rows: a layer's buffers are as wide as the layer needs
-            HY_TRY(linear_t<D>(e, e->h, W, L.w_in_dev, e->proj, nin, rows, nin, W, 0, 1.f, nullptr, 0, st));
+            bool act_done = false;
+            const BranchTail act = plain_act<D>(e, L, nmix, ldcat, HV);
+            HY_TRY(linear_t<D>(e, e->h, W, L.w_in_dev, e->proj, nin, rows, nin, W, 0, 1.f, nullptr, 0, st, 1, 0, 0, 0, nullptr, nullptr, nullptr, nullptr,
+                               act.h ? &act : nullptr, &act_done));
             HY_TRY(mixer_t<D>(e, ri, m, sh, nin, ldcat));
-            if (L.ff > 0) HY_TRY(ff_act_t<D>(e, L, rows, nin, nmix, ldcat, HV));
+            if (L.ff > 0 && !act_done) HY_TRY(ff_act_t<D>(e, L, rows, nin, nmix, ldcat, HV));
             // x += m * ([mixer out ; ff act] . [W_o | W_down]^T)
             HY_TRY(linear_t<D>(e, e->cat, ldcat, L.w_out_dev, e->x, W, rows, W, HV + L.ff, 1, c.residual_mult, nullptr, 0, st));
         } else {

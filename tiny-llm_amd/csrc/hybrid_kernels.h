@@ -35,22 +35,9 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
 }
 
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
-__device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); }
 // SiLU through the hardware's exponential and reciprocal (relative error of a few 1e-7), where every workgroup that reads a row forms it again
 __device__ __forceinline__ float silu_hw(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 __device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
-__device__ __forceinline__ float act_f(float z, int kind) {
-    if (kind == 0) return 0.5f * z * (1.f + erff(z * 0.70710678118654752440f));
-    if (kind == 1) {  // 0.5 z (1 + tanh u) = z / (1 + exp(-2 u)), u = sqrt(2/pi) (z + 0.044715 z^3): one exponential instead of tanhf
-        const float u = 0.79788456080286535588f * (z + 0.044715f * z * z * z);
-        return z / (1.f + expf(-2.f * u));
-    }
-    if (kind == 3) {
-        const float r = fmaxf(z, 0.f);
-        return r * r;
-    }
-    return silu_f(z);
-}
 // a query's temperature at position pos: 1 + coef ln(floor((pos + 1) / every) + 1); coef 0: 1
 __device__ __forceinline__ float q_temperature(int pos, float coef, float every) {
     return coef == 0.f ? 1.f : 1.f + coef * logf((float)floor((double)(pos + 1) / (double)every) + 1.f);
@@ -146,6 +133,7 @@ struct BranchTail {
     const float *bias = nullptr, *pw = nullptr, *pb = nullptr, *ls = nullptr, *add = nullptr, *vec = nullptr, *nw = nullptr, *nb = nullptr;
     float palpha = 0.f, mult = 1.f, nalpha = 0.f;
     void *h = nullptr;
+    int act_from = 0, act_kind = 0, act_ld = 0;  // EPI 6
 };
 template <typename D>
 __device__ __forceinline__ void branch_tail(const BranchTail &t, size_t i, int n, float y) {
@@ -167,6 +155,14 @@ __device__ __forceinline__ void product_out(float *out, int ldc, int N, int m, i
     else if constexpr (EPI == 2) *o = v + bias[n];
     else if constexpr (EPI == 3) *o += alpha * bias[n] * v;
     else if constexpr (EPI == 5) branch_tail<D>(tail, (size_t)m * N + n, n, v);
+    else if constexpr (EPI == 6) {  // columns from act_from on: the feed-forward's, activated and rounded where its second product reads them (ff_act_kernel's terms)
+        if (n < tail.act_from) *o = v;
+        else {
+            const int c = n - tail.act_from;
+            if (tail.bias) v += tail.bias[c];
+            reinterpret_cast<typename D::storage *>(tail.h)[(size_t)m * tail.act_ld + c] = D::from_float(act_f(v, tail.act_kind));
+        }
+    }
     else {
         const float xn = *o + alpha * bias[n] * v;
         *o = xn;
