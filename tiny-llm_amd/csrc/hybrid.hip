@@ -1201,7 +1201,7 @@ static int forward_t(tl_hybrid *e, const Meta &m, const StepShape &sh) {
 
 // final norm on the wanted rows, head product, argmax (and the slots' next input tokens)
 template <typename D>
-static int head_t(tl_hybrid *e, const Meta &m, int n_want, bool set_pending) {
+static int head_t(tl_hybrid *e, const Meta &m, int n_want, bool set_pending, const StepEnd &end) {
     const tl_hybrid_config &c = e->cfg;
     if (n_want <= 0) return TL_OK;
     HY_TRY(norm_t<D>(e, c.final_norm_kind, c.final_norm_dev, c.final_norm_bias_dev, c.final_norm_alpha, c.final_norm_offset, e->hsel, m.want_rows, n_want));
@@ -1213,7 +1213,7 @@ static int head_t(tl_hybrid *e, const Meta &m, int n_want, bool set_pending) {
         TL_CHECK_LAUNCH("hybrid logit scale");
     }
     hipLaunchKernelGGL(argmax_kernel, dim3(n_want), dim3(1024), 0, e->stream, e->logits, c.vocab, e->argmax_dev, set_pending ? m.want_slot : (const int32_t *)nullptr,
-                       e->pending_dev);
+                       e->pending_dev, end);
     TL_CHECK_LAUNCH("hybrid argmax");
     return TL_OK;
 }
@@ -1221,8 +1221,8 @@ static int head_t(tl_hybrid *e, const Meta &m, int n_want, bool set_pending) {
 static int forward(tl_hybrid *e, const Meta &m, const StepShape &sh) {
     return e->cfg.dtype == TL_HY_BF16 ? forward_t<BF16>(e, m, sh) : forward_t<F32>(e, m, sh);
 }
-static int head(tl_hybrid *e, const Meta &m, int n_want, bool set_pending) {
-    return e->cfg.dtype == TL_HY_BF16 ? head_t<BF16>(e, m, n_want, set_pending) : head_t<F32>(e, m, n_want, set_pending);
+static int head(tl_hybrid *e, const Meta &m, int n_want, bool set_pending, const StepEnd &end = StepEnd{}) {
+    return e->cfg.dtype == TL_HY_BF16 ? head_t<BF16>(e, m, n_want, set_pending, end) : head_t<F32>(e, m, n_want, set_pending, end);
 }
 
 static int sync_table(tl_hybrid *e) {
@@ -1775,13 +1775,10 @@ static int decode_steps(tl_hybrid *e, int n_seqs, const int *slots, int steps, i
     HY_TRY(sync_table(e));
     auto one_step = [&]() -> int {
         hipLaunchKernelGGL(decode_meta_kernel, dim3((n_seqs + 63) / 64), dim3(64), 0, e->stream, e->dmeta.seq_slot, n_seqs, e->pending_dev, e->ctx_dev,
-                           e->dmeta.tokens, e->dmeta.row_pos, e->dmeta.seq_prev, e->last_tok_dev, 0, e->hist_dev, e->hist_at_dev, c.max_slots);
+                           e->dmeta.tokens, e->dmeta.row_pos, e->dmeta.seq_prev, e->last_tok_dev);
         TL_CHECK_LAUNCH("hybrid decode meta");
         HY_TRY(forward(e, e->dmeta, sh));
-        HY_TRY(head(e, e->dmeta, n_seqs, true));
-        hipLaunchKernelGGL(decode_meta_kernel, dim3((n_seqs + 63) / 64), dim3(64), 0, e->stream, e->dmeta.seq_slot, n_seqs, e->pending_dev, e->ctx_dev,
-                           e->dmeta.tokens, e->dmeta.row_pos, e->dmeta.seq_prev, e->last_tok_dev, 1, e->hist_dev, e->hist_at_dev, c.max_slots);
-        TL_CHECK_LAUNCH("hybrid decode advance");
+        HY_TRY(head(e, e->dmeta, n_seqs, true, StepEnd{e->ctx_dev, e->hist_dev, e->hist_at_dev, c.max_slots}));
         return TL_OK;
     };
     const bool graph = use_graph && !e->trace;
