@@ -52,6 +52,11 @@ def test_mid_product(dtype, M, N, K):
     _product(dtype, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(192, 33, 256), (250, 64, 520), (1000, 130, 72), (1000, 1984, 136), (1000, 2047, 136)])  # (the last: 512 tiles of 64 x 64)
+def test_mid_product_of_many_rows(M, N, K):
+    _product("float32", M, N, K)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n", [17, 40, 70])
 def test_products_that_split_their_sums_over_workgroups(n, dtype):

@@ -261,7 +261,9 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
         else if (epi == 2) HY_GEMM_ROWS_C(2);
         else if (!with_tail) HY_GEMM_ROWS_C(3);
         else HY_GEMM_ROWS_C(4);
-    } else if (force == 0 && vec_ok && M < 192) {
+    } else if (force == 0 && vec_ok && (M < 192 || (long)((M + 63) / 64) * ((N + 63) / 64) * batch < 2 * qmm3_num_cus())) {
+        // (from 192 rows on what is left is float32 or batched: the 64 x 64 LDS tiles win once they give every CU two -- float32, tiles / straight from memory in us:
+        // 400 x 1,024 of K 5,120 201 / 100, 1,000 x 2,048 of K 10,240 575 / 456, 600 x 4,096 of K 1,024 75 / 69, 1,000 x 4,096 93 / 100, 2,000 x 8,192 of K 2,048 547 / 739)
         // 16 to 64 rows a workgroup; K split over workgroups (at least two 128-byte pieces a wave) until every CU has two, as far as the partial sums' buffer reaches
         const int mt = M > 48 ? 4 : (M > 32 ? 3 : 2), cols = (N + 31) / 32, mtiles = (M + 16 * mt - 1) / (16 * mt), pieces = (K + 128 / (int)sizeof(S) - 1) / (128 / (int)sizeof(S));
         int sk = 1;
