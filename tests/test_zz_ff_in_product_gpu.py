@@ -1,4 +1,4 @@
-"""GPU tier: the plain feed-forward's activation as the end of the product that forms its columns -- rows, split sums, 256-wide and 128-wide tiles -- against
+"""GPU tier: the plain feed-forward's activation as the end of the product that forms its columns (rows, split sums, tiles) or behind it (large bf16 prompts), against
 the float64 restatement of tests/layer_list_oracle.py: beside the mixer's columns (Fonapel) and of its own matrices with a bias (Vabuzen); widths that come in
 fours and widths that do not.  The whole list's logits, tolerances of the families' own tests."""
 

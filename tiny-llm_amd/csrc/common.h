@@ -216,19 +216,4 @@ int paged_attention_packed(const uint16_t *q, const void *key_pages, const void 
 
 inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 
-// activations by number: 0 gelu (erf), 1 gelu (tanh), 2 silu, 3 squared relu
-__device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); }
-__device__ __forceinline__ float act_f(float z, int kind) {
-    if (kind == 0) return 0.5f * z * (1.f + erff(z * 0.70710678118654752440f));
-    if (kind == 1) {  // 0.5 z (1 + tanh u) = z / (1 + exp(-2 u)), u = sqrt(2/pi) (z + 0.044715 z^3): one exponential instead of tanhf
-        const float u = 0.79788456080286535588f * (z + 0.044715f * z * z * z);
-        return z / (1.f + expf(-2.f * u));
-    }
-    if (kind == 3) {
-        const float r = fmaxf(z, 0.f);
-        return r * r;
-    }
-    return silu_f(z);
-}
-
 }  // namespace tl

@@ -32,14 +32,10 @@ struct Gemm8Args {
     int M, N, K;
     float *out_f32 = nullptr;  // EPI_F32_STORE / EPI_F32_AXPY: [M, N] float32 (a float32 residual stream or float32 projections behind bf16 operands)
     float alpha = 1.f;         // EPI_F32_AXPY: out_f32 += alpha * product
-    // EPI_F32_ACT: columns below act_from go to out_f32, the others as bf16(act(product + act_bias)) to act_out, rows of act_ld (act_from, act_ld multiples of 4)
-    uint16_t *act_out = nullptr;
-    const float *act_bias = nullptr;
-    int act_from = 0, act_ld = 0, act_kind = 0;
     const float *col_scale = nullptr;  // EPI_F32_AXPY, optional [N]: out_f32 += alpha * col_scale[n] * product (a per-channel scale of the branch)
 };
 // epilogues beside EPI_STORE / EPI_RESIDUAL / EPI_SWIGLU (qmv.h): the accumulators leave as float32
-enum { EPI_F32_STORE = 3, EPI_F32_AXPY = 4, EPI_F32_ACT = 5 };
+enum { EPI_F32_STORE = 3, EPI_F32_AXPY = 4 };
 
 constexpr int G8_BK = 64, G8_WAVES = 8;
 #ifdef G8_TRACE  // tools/lab/gemm8_lab only: wall-clock stamps of wave 0 of workgroup G8_TRACE behind every step's barrier (and around a tile's epilogue)

@@ -210,12 +210,7 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
             Gemm8Args g{};
             g.a = (const uint16_t *)A, g.w = (const uint16_t *)W, g.M = M, g.N = N, g.K = K, g.out_f32 = out, g.alpha = alpha;
             if (epi == 3) g.col_scale = bias;
-            const bool act8 = act && epi == 0 && act->act_from % 4 == 0 && act->act_ld % 4 == 0 && ((uintptr_t)act->bias % 16 | (uintptr_t)act->h % 8) == 0;
-            if (act8) {
-                g.act_out = (uint16_t *)act->h, g.act_bias = act->bias, g.act_from = act->act_from, g.act_ld = act->act_ld, g.act_kind = act->act_kind;
-                *act_done = true;
-            }
-            if (launch_gemm8_bf16(g, act8 ? EPI_F32_ACT : ((epi == 1 || epi == 3) ? EPI_F32_AXPY : EPI_F32_STORE), st) == 0) {
+            if (launch_gemm8_bf16(g, (epi == 1 || epi == 3) ? EPI_F32_AXPY : EPI_F32_STORE, st) == 0) {  // (an activation follows: see plain_act)
                 if (epi == 2) {
                     const size_t n = (size_t)M * N;
                     hipLaunchKernelGGL(add_rowvec_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, out, bias, N, M);
@@ -224,7 +219,6 @@ static int linear_t(const tl_hybrid *e, const void *A, int lda, const void *W, f
                 return TL_OK;
             }
         }
-        if (act_done) *act_done = false;
         TL_REQUIRE(force != 3, "hybrid linear: the 256-wide tile GEMM does not take this shape");
     }
     const bool with_tail = tail && tail->out && epi == 3 && batch == 1 && ldc == N;
@@ -949,7 +943,8 @@ static int ff_act_t(tl_hybrid *e, const tl_hybrid_layer &L, int rows, int ldp, i
 }
 
 // The activation of a feed-forward without gates or experts leaves with the product that forms its columns (from `up0` on), into cat: one launch and a float32
-// round trip of those columns less (2,048 rows x 8,192: 17 us of their own; a step of four rows 3 us).  h NULL: ff_act_t behind the product.
+// round trip of those columns less (3 us a layer in a step of four rows).  Not with the tile GEMM of large prompts: its one workgroup a CU has no other work
+// beside the epilogue's exponentials (2,048 x 16,416 of K 2,048: 25 us more, ff_act_kernel 17 us).  h NULL: ff_act_t behind the product.
 template <typename D>
 static BranchTail plain_act(const tl_hybrid *e, const tl_hybrid_layer &L, int up0, int ldcat, int col0) {
     BranchTail t;

@@ -35,9 +35,22 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
 }
 
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
+__device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); }
 // SiLU through the hardware's exponential and reciprocal (relative error of a few 1e-7), where every workgroup that reads a row forms it again
 __device__ __forceinline__ float silu_hw(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 __device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+__device__ __forceinline__ float act_f(float z, int kind) {
+    if (kind == 0) return 0.5f * z * (1.f + erff(z * 0.70710678118654752440f));
+    if (kind == 1) {  // 0.5 z (1 + tanh u) = z / (1 + exp(-2 u)), u = sqrt(2/pi) (z + 0.044715 z^3): one exponential instead of tanhf
+        const float u = 0.79788456080286535588f * (z + 0.044715f * z * z * z);
+        return z / (1.f + expf(-2.f * u));
+    }
+    if (kind == 3) {
+        const float r = fmaxf(z, 0.f);
+        return r * r;
+    }
+    return silu_f(z);
+}
 // a query's temperature at position pos: 1 + coef ln(floor((pos + 1) / every) + 1); coef 0: 1
 __device__ __forceinline__ float q_temperature(int pos, float coef, float every) {
     return coef == 0.f ? 1.f : 1.f + coef * logf((float)floor((double)(pos + 1) / (double)every) + 1.f);
