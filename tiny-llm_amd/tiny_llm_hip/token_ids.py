@@ -7,8 +7,8 @@ from typing import Sequence
 
 def token_ids(tokens: Sequence[int]) -> array:
     """The ids as an array of int32.  Lists and tuples of integers convert in one pass of C (2,048 ids: 34 us; one by one, as a list and into
-    a ctypes array, 310 us); anything else --
-    other sequences, floats, tensors, ids past 32 bits, which wrap as a ctypes array wraps them -- goes element by element through int()."""
+    a ctypes array, 310 us); anything else -- other sequences, floats, tensors, ids past 32 bits, which wrap as a ctypes array wraps them -- goes
+    element by element through int()."""
     if isinstance(tokens, array) and tokens.typecode == "i":
         return tokens
     if isinstance(tokens, (list, tuple)):
